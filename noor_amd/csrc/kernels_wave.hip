@@ -46,6 +46,7 @@ constexpr uint32_t kNoItem = 0xFFFFFFFFu;
 constexpr int kIters = 6;
 constexpr uint64_t kMaxGroupItems = 1ull << 28;  // sample-buffer entries per group of layers (4.3 GB)
 constexpr int kRefill = 32;  // idle lanes of a wave that trigger a refill from the ray queue
+constexpr uint32_t kMinChunk = 48, kMaxChunk = 256;  // queue entries one atomic claims for a wave (refill)
 constexpr uint32_t kDrainMax = 1u << 20;  // paths in flight at which k_drain finishes a group
 constexpr uint32_t kMaxAutoPool = 1u << 25;  // path slots of an automatic pool, at most
 
@@ -104,7 +105,7 @@ struct WavePool {
     uint32_t capacity = 0;
     int block = 64;
     int stack_lds = 0;
-    int steps = 32;            // traversal steps between refills of the persistent kernels
+    int steps = 20;            // traversal steps between refills of the persistent kernels
     uint32_t sb_items = 0;     // sample buffer entries
     uint32_t max_views = 0, max_segments = 0;
     // path state (one slot per path in flight)
@@ -364,24 +365,58 @@ __global__ void k_regen(const DevScene* __restrict__ Sp, WavePool B, int cur) {
     B.qd[cur][c0 + t] = make_float4(r.d.x, r.d.y, r.d.z, 0.0f);
 }
 
+// The part of a queue that a persistent wave has claimed and not yet handed to
+// its lanes (wave-uniform).
+struct Claim {
+    uint32_t next, end;
+    bool done;  // nothing is left in the claim or in the queue
+};
+
 // Refill of a persistent wave: when at least kRefill lanes are idle (or all
-// are), one atomic hands the idle lanes consecutive queue entries.  Returns
-// this lane's entry, or UINT32_MAX.  `exhausted` becomes true (wave-uniform)
-// once the queue has run out.
-__device__ __forceinline__ uint32_t refill(uint32_t* work, uint32_t count, bool have, bool& exhausted) {
-    if (exhausted) return 0xFFFFFFFFu;
+// are), the idle lanes take consecutive entries of the wave's claim; when it
+// runs out, one atomic claims the next chunk of the queue.  Returns this lane's
+// entry, or UINT32_MAX.
+//
+// One atomic per refill bounded the traversal kernels: 64 rays at most per
+// returning atomic on one address, 11 ns each, is 5.7 G rays/s for the whole
+// GPU, and k_extend ran at 5.2 G rays/s on the 1M-triangle scene (1080p, 64
+// spp).  With chunks of 256 it takes 12.9 ms of that film instead of 29.0, on
+// the 5M-triangle terrain (32 spp) 22.6 instead of 25.9.  Chunks of 128 are
+// still at the atomics' rate (17.8 ms), chunks of 512 widen the part of the
+// scene in flight (13.3 and 23.2 ms).  A chunk shrinks to the wave's 1/DIV
+// share of what was left at its last claim, so that no wave sits on rays while
+// others idle: fixed chunks of 256 took 4.7 ms of the 512x512 box's film
+// against 4.1, and 64 as the least 3.0 against 2.9 ms of a 200k-pixel film.
+// The closest-hit rays measured best with 1/2 of the share; the fewer and
+// longer occlusion rays with 1/4 (9.4 against 9.8 ms on the terrain).
+template <uint32_t DIV>
+__device__ __forceinline__ uint32_t refill(uint32_t* work, uint32_t count, bool have, Claim& c) {
+    if (c.done) return 0xFFFFFFFFu;
     const unsigned long long idle = __ballot(!have);
-    const int n = __popcll(idle);
-    if (n < kRefill && n < 64) return 0xFFFFFFFFu;
-    const uint32_t lane = lane_id();
-    const int leader = __ffsll((long long)idle) - 1;
-    uint32_t base = 0;
-    if ((int)lane == leader) base = atomicAdd(work, (uint32_t)n);
-    base = __shfl(base, leader, 64);
-    if (base + (uint32_t)n >= count) exhausted = true;
-    if (have) return 0xFFFFFFFFu;
-    const uint32_t idx = base + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-    return idx < count ? idx : 0xFFFFFFFFu;
+    const uint32_t n = (uint32_t)__popcll(idle);
+    if (n < (uint32_t)kRefill) return 0xFFFFFFFFu;
+    const uint32_t lane = lane_id(), rank = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+    const uint32_t avail = c.end - c.next;
+    uint32_t idx = c.next + rank;
+    bool valid = rank < avail;
+    if (avail >= n) {
+        c.next += n;
+    } else {
+        const uint32_t need = n - avail;
+        const uint32_t share = (count - c.end) / (gridDim.x * (blockDim.x >> 6) * DIV);
+        const uint32_t chunk = max(min(share, kMaxChunk), max(need, kMinChunk));
+        uint32_t base = 0;
+        if (lane == 0) base = atomicAdd(work, chunk);
+        base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+        c.end = min(base + chunk, count);
+        c.next = min(base + need, c.end);
+        if (!valid) {
+            idx = base + (rank - avail);
+            valid = idx < c.end;
+        }
+    }
+    c.done = c.next >= c.end && c.end >= count;
+    return !have && valid ? idx : 0xFFFFFFFFu;
 }
 
 // Held to 80 VGPRs (six waves per SIMD, a few spilled registers): measured 6%
@@ -396,12 +431,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
     const uint32_t count = ctl->ray_count[cur] + ctl->new_rays[cur];
     const uint32_t* q = B.q_ray[cur];
     Counters cnt{0, 0, 0, 0};
-    bool overflow = false, have = false, exhausted = false;
+    bool overflow = false, have = false;
+    Claim claim{0u, 0u, count == 0u};
     uint32_t ext = 0, nhit = 0;  // rays this lane started, and (STATS) how many hit
     uint32_t p = 0, qi = 0;
     ClosestTrav t;
     for (;;) {
-        const uint32_t idx = refill(&ctl->work_extend.v, count, have, exhausted);
+        const uint32_t idx = refill<2>(&ctl->work_extend.v, count, have, claim);
         if (idx != 0xFFFFFFFFu) {
             p = q[idx];
             const float4 o = B.qo[cur][idx], d = B.qd[cur][idx];
@@ -651,7 +687,8 @@ __global__ void k_shadow(const DevScene* __restrict__ Sp, WavePool B, DevStats* 
     const TravStack st = make_stack(S, smem);
     const uint32_t count = ctl->shadow_count;
     Counters cnt{0, 0, 0, 0};
-    bool overflow = false, have = false, exhausted = false;
+    bool overflow = false, have = false;
+    Claim claim{0u, 0u, count == 0u};
     uint32_t shd = 0;  // rays this lane started
     uint32_t p = 0;
     // a task is one path's NEE: its light-sampled ray (a), then, with MIS,
@@ -659,7 +696,7 @@ __global__ void k_shadow(const DevScene* __restrict__ Sp, WavePool B, DevStats* 
     bool second = false, occ_a = false;
     AnyTrav t;
     for (;;) {
-        const uint32_t idx = refill(&ctl->work_shadow.v, count, have, exhausted);
+        const uint32_t idx = refill<4>(&ctl->work_shadow.v, count, have, claim);
         if (idx != 0xFFFFFFFFu) {
             p = B.q_shadow[idx];
             occ_a = false;
