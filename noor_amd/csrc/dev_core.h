@@ -237,15 +237,45 @@ __device__ __forceinline__ float rng_next(Rng& r, int kind) {
 struct Ray {
     f3 o, d, inv;
     float tmax;
-    uint32_t pn;  // bit a set when d[a] <= 0 (the reference posneg); bit 3: box4_hit's fast form applies
+    uint32_t pn;  // bit a set when d[a] <= 0 (the reference posneg); bit 3: box4_hit's fast form applies;
+                  // bit 4: no quotient of two components of d leaves the normal numbers
     int kx, ky, kz;
     float Sx, Sy, Sz;
 };
 
+// 1 / x, correctly rounded as the IEEE division is, in half its instructions:
+// one fused Newton step on the hardware reciprocal gives the same bits for
+// every x whose hardware reciprocal is a normal number (all 2^32 values
+// compared with 1.0f / x on MI355X); the others take the division.
+__device__ __forceinline__ bool is_normal(float x) { return __builtin_isfpclass(x, 0x108); }
+__device__ __forceinline__ float rcp_step(float x, float y) { return __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y); }
+__device__ __forceinline__ float frcp(float x) {
+    const float y = __builtin_amdgcn_rcpf(x);
+    return is_normal(y) ? rcp_step(x, y) : 1.0f / x;
+}
+// a / b, correctly rounded, from y = 1 / b correctly rounded, where no step
+// leaves the normal numbers: the first correction makes q faithful, the second
+// then rounds correctly (Markstein, "Computation of elementary functions on the
+// IBM RISC System/6000 processor", IBM J. Res. Dev. 34(1), 1990).
+__device__ __forceinline__ float div_by_rcp(float a, float b, float y) {
+    float q = a * y;
+    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+
 // Box-test terms of a ray: reciprocal direction and octant flags.
 __device__ __forceinline__ void ray_update_box(Ray& r) {
-    r.inv = f3{1.0f / r.d.x, 1.0f / r.d.y, 1.0f / r.d.z};
     r.pn = (r.d.x > 0.0f ? 0u : 1u) | (r.d.y > 0.0f ? 0u : 2u) | (r.d.z > 0.0f ? 0u : 4u);
+    const f3 y = f3{__builtin_amdgcn_rcpf(r.d.x), __builtin_amdgcn_rcpf(r.d.y), __builtin_amdgcn_rcpf(r.d.z)};
+    const float hi = fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fabsf(y.z));
+    const float lo = fminf(fminf(fabsf(y.x), fabsf(y.y)), fabsf(y.z));
+    if (hi <= 0x1p60f && lo >= 0x1p-60f) {
+        // frcp, with one range check for the three
+        r.inv = f3{rcp_step(r.d.x, y.x), rcp_step(r.d.y, y.y), rcp_step(r.d.z, y.z)};
+        r.pn |= 24u;
+        return;
+    }
+    r.inv = f3{1.0f / r.d.x, 1.0f / r.d.y, 1.0f / r.d.z};
     // the fast slab form needs finite reciprocals whose products with a
     // node's step cannot overflow (steps stay far below 2^40)
     const float mi = fmaxf(fmaxf(fabsf(r.inv.x), fabsf(r.inv.y)), fabsf(r.inv.z));
@@ -276,9 +306,15 @@ __device__ __forceinline__ void ray_update_tri(Ray& r) {
     r.ky = ky;
     r.kz = kz;
     const float dz = c3(r.d, kz);
-    r.Sx = c3(r.d, kx) / dz;
-    r.Sy = c3(r.d, ky) / dz;
     r.Sz = c3(r.inv, kz);  // 1 / dz, already rounded once in inv
+    const float dx = c3(r.d, kx), dy = c3(r.d, ky);
+    if (r.pn & 16u) {
+        r.Sx = div_by_rcp(dx, dz, r.Sz);
+        r.Sy = div_by_rcp(dy, dz, r.Sz);
+    } else {
+        r.Sx = dx / dz;
+        r.Sy = dy / dz;
+    }
 }
 
 __device__ __forceinline__ void ray_update(Ray& r) {
@@ -431,10 +467,11 @@ __device__ __forceinline__ uint32_t box4_hit(const Ray& r, const WideNode& n, fl
         const float ty1 = __builtin_fmaf((float)((fy >> (8 * c)) & 0xFFu), By, Ay);
         const float tz0 = __builtin_fmaf((float)((nz >> (8 * c)) & 0xFFu), Bz, Az);
         const float tz1 = __builtin_fmaf((float)((fz >> (8 * c)) & 0xFFu), Bz, Az);
+        // entered if t0 <= t1, t1 >= 0 and t0 <= tmaxs
         const float t0 = fmaxf(fmaxf(tx0, ty0), tz0) - W;
-        const float t1 = fminf(fminf(tx1, ty1), tz1) * BOX_SLACK + W;
+        const float t1 = __builtin_fmaf(fminf(fminf(tx1, ty1), tz1), BOX_SLACK, W);
         tn[c] = t0;
-        if (t0 <= t1 && t0 <= tmaxs && t1 >= 0.0f) mask |= 1u << c;
+        if (fmaxf(t0, 0.0f) <= t1 && t0 <= tmaxs) mask |= 1u << c;
     }
     return mask & (meta >> 24);
 }
@@ -501,7 +538,7 @@ __device__ __forceinline__ bool tri_watertight(const DevScene& S, const Ray& r, 
     if (det == 0.0f) return false;
     const float Az = r.Sz * Az0, Bz = r.Sz * Bz0, Cz = r.Sz * Cz0;
     const float Tt = U * Az + V * Bz + W * Cz;
-    const float inv = 1.0f / det;
+    const float inv = frcp(det);
     const float t = Tt * inv;
     if (!(t >= 0.0f) || t > r.tmax) return false;
     to = t;
@@ -644,18 +681,20 @@ __device__ __forceinline__ void cswap(float& a, float& b, uint32_t& ra, uint32_t
     rb = ub;
 }
 
-// Two-level closest hit (noor/cuda/bvh.cuh:142-191) over the wide BVH, as a
-// resumable state machine: closest_steps() advances a traversal by at most
-// `max_steps` node or leaf visits and returns true when it has finished, so a
-// persistent kernel can hand a finished lane a new ray while the others go
-// on.  Ties in t are broken by (prim_id, instance); light nodes win only when
-// strictly closer.  Hit children are followed nearest first.
+// Two-level closest hit (noor/cuda/bvh.cuh:142-191) and any hit
+// (noor/cuda/bvh.cuh:193-234) over the wide BVH, as a resumable state machine:
+// trav_steps() advances a traversal by at most `max_steps` node or leaf visits
+// and returns true when it has finished, so a persistent kernel can hand a
+// finished lane a new ray while the others go on.  Ties in t are broken by
+// (prim_id, instance); light nodes win only when strictly closer.  Hit children
+// are followed nearest first, by occlusion rays too (in slot order those took
+// 3% longer on the 1080p terrain, as long elsewhere).
 // The world ray is kept as origin and direction only; lray is the ray of the
 // level being traversed (world, or object space inside an instance) with its
 // precomputed terms and the current closest distance, and is rebuilt from the
 // world ray on the way back to the top level.  Keeping one full Ray instead of
 // two saves the registers that decide how many waves a CU can keep in flight.
-struct ClosestTrav {
+struct Trav {
     f3 o, d;
     Ray lray;
     uint32_t cur, ins;
@@ -664,7 +703,7 @@ struct ClosestTrav {
     Hit h;
 };
 
-__device__ __forceinline__ void closest_begin(const DevScene& S, const Ray& r, ClosestTrav& t) {
+__device__ __forceinline__ void trav_begin(const DevScene& S, const Ray& r, Trav& t) {
     t.o = r.o;
     t.d = r.d;
     t.lray = r;
@@ -695,9 +734,13 @@ __device__ __forceinline__ uint32_t leaf_next(uint32_t cur) {
     return ((cur >> REF_LEAF_COUNT_SHIFT) & 7u) ? cur + 1u - (1u << REF_LEAF_COUNT_SHIFT) : REF_EMPTY;
 }
 
-template <bool STATS, bool ALPHA = false>
-__device__ __forceinline__ bool closest_steps(const DevScene& S, ClosestTrav& t, const TravStack& st, Counters& c,
-                                              bool& overflow, int max_steps) {
+//
+// KIND: a closest-hit query, an any-hit one (ends at the first triangle or light
+// it finds, t.hit), or the lane's choice in `any`.
+enum : int { TRAV_CLOSEST, TRAV_ANY, TRAV_MIXED };
+template <bool STATS, bool ALPHA, int KIND>
+__device__ __forceinline__ bool trav_steps(const DevScene& S, Trav& t, const TravStack& st, Counters& c,
+                                           bool& overflow, int max_steps, bool any = KIND == TRAV_ANY) {
     for (int step = 0; step < max_steps; ++step) {
         const uint32_t cur = t.cur;
         const uint32_t kind = (cur >> REF_KIND_SHIFT) & 3u;
@@ -746,6 +789,10 @@ __device__ __forceinline__ bool closest_steps(const DevScene& S, ClosestTrav& t,
             const uint32_t ti = cur & REF_LEAF_START_MASK;
             float tt, u, v;
             if (tri_test<STATS, ALPHA>(S, t.lray, ti, tt, u, v, c)) {
+                if (KIND != TRAV_CLOSEST && any) {
+                    t.hit = true;
+                    return true;
+                }
                 const uint32_t key = ldg(S.prim_ids + ti);
                 bool take = false;
                 if (tt < t.lray.tmax) take = true;
@@ -774,7 +821,13 @@ __device__ __forceinline__ bool closest_steps(const DevScene& S, ClosestTrav& t,
             // light nodes are top-level references: lray is the world ray here
             const uint32_t li = cur & REF_INDEX_MASK;
             Ray tr = t.lray;
-            if (light_node_intersect(S, li, tr) && tr.tmax < t.lray.tmax) {
+            const bool lh = light_node_intersect(S, li, tr);
+            if (KIND != TRAV_CLOSEST && any) {
+                if (lh) {
+                    t.hit = true;
+                    return true;
+                }
+            } else if (lh && tr.tmax < t.lray.tmax) {
                 t.lray.tmax = tr.tmax;
                 t.hit = true;
                 t.h.t = tr.tmax;
@@ -794,108 +847,23 @@ __device__ __forceinline__ bool closest_steps(const DevScene& S, ClosestTrav& t,
 template <bool STATS, bool ALPHA = false>
 __device__ __forceinline__ bool bvh_closest(const DevScene& S, Ray& ray, Hit& h, const TravStack& st, Counters& c,
                                             bool& overflow) {
-    ClosestTrav t;
-    closest_begin(S, ray, t);
-    while (!closest_steps<STATS, ALPHA>(S, t, st, c, overflow, 1 << 30)) {
+    Trav t;
+    trav_begin(S, ray, t);
+    while (!trav_steps<STATS, ALPHA, TRAV_CLOSEST>(S, t, st, c, overflow, 1 << 30)) {
     }
     ray.tmax = t.lray.tmax;
     h = t.h;
     return t.hit;
 }
 
-// Any hit (noor/cuda/bvh.cuh:193-234) over the wide BVH, resumable like the
-// closest-hit traversal.
-struct AnyTrav {
-    f3 o, d;  // world ray; lray as in ClosestTrav (tmax fixed)
-    Ray lray;
-    uint32_t cur;
-    int sp;
-    bool occluded, world;
-};
-
-__device__ __forceinline__ void any_begin(const DevScene& S, const Ray& r, AnyTrav& t) {
-    t.o = r.o;
-    t.d = r.d;
-    t.lray = r;
-    t.world = true;
-    t.cur = S.wroot;
-    t.sp = 0;
-    t.occluded = false;
-}
-
-// Steps as in closest_steps (one node, triangle, instance or light per step).
-template <bool STATS, bool ALPHA = false>
-__device__ __forceinline__ bool any_steps(const DevScene& S, AnyTrav& t, const TravStack& st, Counters& c,
-                                          bool& overflow, int max_steps) {
-    for (int step = 0; step < max_steps; ++step) {
-        const uint32_t cur = t.cur;
-        const uint32_t kind = (cur >> REF_KIND_SHIFT) & 3u;
-        if (kind == REF_INST || ((cur & REF_TLAS) && !t.world)) {
-            f3 o = t.o, d = t.d;
-            if (kind == REF_INST) {
-                if (STATS) c.inst++;
-                const Xf T = xf_load(S.xf + 9 * (size_t)(cur & REF_INDEX_MASK));
-                o = xf_pt(T, t.o);
-                d = xf_vec(T, t.d);
-            }
-            t.lray.o = o;
-            t.lray.d = d;
-            ray_update_box(t.lray);
-            if (kind == REF_INST) ray_update_tri(t.lray);  // the top level holds no triangles
-            t.world = kind != REF_INST;
-        }
-        if (kind == REF_INNER) {
-            if (STATS) c.nodes++;
-            const WideNode n = load_wnode(S, cur & REF_INDEX_MASK);
-            float tn[4];
-            uint32_t m = box4_hit(t.lray, n, tn);
-            if (m != 0u) {
-                const int k = __popc(m);
-                if (t.sp + k - 1 > st.depth) {
-                    overflow = true;
-                    return true;
-                }
-                const uint4 rf = n.ref();
-                t.cur = ref_of(rf, __ffs(m) - 1);
-                m &= m - 1u;
-                while (m) {
-                    st.put(t.sp++, ref_of(rf, __ffs(m) - 1));
-                    m &= m - 1u;
-                }
-                continue;
-            }
-        } else if (kind == REF_LEAF) {
-            float tt, u, v;
-            if (tri_test<STATS, ALPHA>(S, t.lray, cur & REF_LEAF_START_MASK, tt, u, v, c)) {
-                t.occluded = true;
-                return true;
-            }
-            t.cur = leaf_next(cur);
-            if (t.cur != REF_EMPTY) continue;
-        } else if (kind == REF_INST) {
-            t.cur = ldg(S.inst_root + (cur & REF_INDEX_MASK));
-            if (t.cur != REF_EMPTY) continue;
-        } else {
-            Ray tr = t.lray;
-            if (light_node_intersect(S, cur & REF_INDEX_MASK, tr)) {
-                t.occluded = true;
-                return true;
-            }
-        }
-        if (t.sp == 0) return true;
-        t.cur = st.get(--t.sp);
-    }
-    return false;
-}
-
 template <bool STATS, bool ALPHA = false>
 __device__ __forceinline__ bool bvh_any(const DevScene& S, const Ray& ray, const TravStack& st, Counters& c,
                                         bool& overflow) {
-    AnyTrav t;
-    any_begin(S, ray, t);
-    while (!any_steps<STATS, ALPHA>(S, t, st, c, overflow, 1 << 30)) {
+    Trav t;
+    trav_begin(S, ray, t);
+    while (!trav_steps<STATS, ALPHA, TRAV_ANY>(S, t, st, c, overflow, 1 << 30)) {
     }
-    return t.occluded;
+    return t.hit;
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -435,19 +435,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
     Claim claim{0u, 0u, count == 0u};
     uint32_t ext = 0, nhit = 0;  // rays this lane started, and (STATS) how many hit
     uint32_t p = 0, qi = 0;
-    ClosestTrav t;
+    Trav t;
     for (;;) {
         const uint32_t idx = refill<2>(&ctl->work_extend.v, count, have, claim);
         if (idx != 0xFFFFFFFFu) {
             p = q[idx];
             const float4 o = B.qo[cur][idx], d = B.qd[cur][idx];
             qi = (idx << 3) | (o.w != 0.0f ? 4u : 0u);
-            closest_begin(S, mkray(f3{o.x, o.y, o.z}, f3{d.x, d.y, d.z}, K_INF), t);
+            trav_begin(S, mkray(f3{o.x, o.y, o.z}, f3{d.x, d.y, d.z}, K_INF), t);
             have = true;
             ++ext;
         }
         if (__ballot(have) == 0ull) break;
-        if (have && closest_steps<STATS, ALPHA>(S, t, st, cnt, overflow, B.steps)) {
+        if (have && trav_steps<STATS, ALPHA, TRAV_CLOSEST>(S, t, st, cnt, overflow, B.steps)) {
             B.hit[2 * (size_t)p] = make_uint4(__float_as_uint(t.h.t), __float_as_uint(t.h.u), __float_as_uint(t.h.v),
                                               t.h.prim);
             B.hit[2 * (size_t)p + 1] = make_uint4(t.h.inst, (t.hit ? t.h.kind : 0u) | qi, 0u, 0u);
@@ -694,7 +694,7 @@ __global__ void k_shadow(const DevScene* __restrict__ Sp, WavePool B, DevStats* 
     // a task is one path's NEE: its light-sampled ray (a), then, with MIS,
     // its BSDF-sampled ray (b), traced one after the other by the same lane
     bool second = false, occ_a = false;
-    AnyTrav t;
+    Trav t;
     for (;;) {
         const uint32_t idx = refill<4>(&ctl->work_shadow.v, count, have, claim);
         if (idx != 0xFFFFFFFFu) {
@@ -702,18 +702,18 @@ __global__ void k_shadow(const DevScene* __restrict__ Sp, WavePool B, DevStats* 
             occ_a = false;
             second = MIS && __float_as_int(B.nee_a[p].w) == 0;  // no light-sampled ray: the BSDF-sampled one only
             const float4 o = second ? B.sh2_o[p] : B.sh_o[idx], d = second ? B.sh2_d[p] : B.sh_d[idx];
-            any_begin(S, mkray(f3{o.x, o.y, o.z}, f3{d.x, d.y, d.z}, o.w), t);
+            trav_begin(S, mkray(f3{o.x, o.y, o.z}, f3{d.x, d.y, d.z}, o.w), t);
             have = true;
             ++shd;
         }
         if (__ballot(have) == 0ull) break;
-        if (have && any_steps<STATS, ALPHA>(S, t, st, cnt, overflow, B.steps)) {
+        if (have && trav_steps<STATS, ALPHA, TRAV_ANY>(S, t, st, cnt, overflow, B.steps)) {
             const bool nb = MIS && B.nee_b[p].w != 0.0f;
             if (!second && nb) {
-                occ_a = t.occluded;
+                occ_a = t.hit;
                 second = true;
                 const float4 o = B.sh2_o[p], d = B.sh2_d[p];
-                any_begin(S, mkray(f3{o.x, o.y, o.z}, f3{d.x, d.y, d.z}, o.w), t);
+                trav_begin(S, mkray(f3{o.x, o.y, o.z}, f3{d.x, d.y, d.z}, o.w), t);
                 ++shd;
                 continue;
             }
@@ -728,8 +728,8 @@ __global__ void k_shadow(const DevScene* __restrict__ Sp, WavePool B, DevStats* 
                 const float4 b = B.nee_b[p];
                 nee.b = f3{b.x, b.y, b.z};
             }
-            const bool oa = nee.na ? (second && nb ? occ_a : t.occluded) : false;
-            const bool ob = nb ? t.occluded : false;
+            const bool oa = nee.na ? (second && nb ? occ_a : t.hit) : false;
+            const bool ob = nb ? t.hit : false;
             PathState ps;
             const float4 L = B.Lb[2 * (size_t)p];
             ps.L = f3{L.x, L.y, L.z};
