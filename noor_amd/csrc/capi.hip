@@ -375,6 +375,7 @@ noor_status noor_create(const noor_payload_view* P, const noor_hosek* hosek, con
     c->bvh_root = P->bvh_root_node;
 
     // four-wide BVH for the traversal kernels
+    std::vector<uint32_t> flat_inst;  // instance of each triangle of a flat mesh
     {
         noor::WideBvh wb;
         const std::string werr = noor::build_wide_bvh(P, wb);
@@ -385,6 +386,8 @@ noor_status noor_create(const noor_payload_view* P, const noor_hosek* hosek, con
         S.stack_depth = (int)c->stack_need;
         S.stack_lds = std::min<int>(S.stack_depth, c->stack_lds);
         S.wroot = wb.root;
+        S.wroot_strict = wb.root_strict;
+        flat_inst = std::move(wb.tri_inst);
         if ((st = dev_upload(c, (noor::QNode**)&S.wbvh, wb.qnodes.data(), wb.qnodes.size())) != NOOR_OK) return bail(st);
         if ((st = dev_upload(c, (uint32_t**)&S.inst_root, wb.inst_root.data(), wb.inst_root.size())) != NOOR_OK)
             return bail(st);
@@ -402,17 +405,23 @@ noor_status noor_create(const noor_payload_view* P, const noor_hosek* hosek, con
     if ((st = dev_upload(c, (noor_uint4**)&S.wald1, P->wald_bnu_bnv_au_av, nt)) != NOOR_OK) return bail(st);
     if ((st = dev_upload(c, (noor_uint4**)&S.wald2, P->wald_cnu_cnv_deg_mat, nt)) != NOOR_OK) return bail(st);
     if ((st = dev_upload(c, (noor_uint4**)&S.attr, P->attribute_indices, nt)) != NOOR_OK) return bail(st);
-    std::vector<uint32_t> ids(nt ? nt : 1);
-    for (uint32_t i = 0; i < nt; ++i) ids[i] = P->prim_ids ? P->prim_ids[i] : i;
-    if ((st = dev_upload(c, (uint32_t**)&S.prim_ids, ids.data(), ids.size())) != NOOR_OK) return bail(st);
     {
-        // watertight records: the three vertices of each triangle in leaf order
+        // the three vertices of each triangle in leaf order, with what a hit needs of it in their fourth words
         std::vector<noor_float4> tri((size_t)3 * (nt ? nt : 1));
+        auto word = [](uint32_t u) {
+            float f;
+            std::memcpy(&f, &u, 4);
+            return f;
+        };
         for (uint32_t i = 0; i < nt; ++i) {
             const noor_uint4 a = P->attribute_indices[i];
-            tri[3 * (size_t)i + 0] = P->vertices[a.x];
-            tri[3 * (size_t)i + 1] = P->vertices[a.y];
-            tri[3 * (size_t)i + 2] = P->vertices[a.z];
+            noor_float4* t = &tri[3 * (size_t)i];
+            t[0] = P->vertices[a.x];
+            t[1] = P->vertices[a.y];
+            t[2] = P->vertices[a.z];
+            t[0].w = word(P->prim_ids ? P->prim_ids[i] : i);
+            t[1].w = word(flat_inst.empty() ? 0u : flat_inst[i]);
+            t[2].w = word(P->wald_cnu_cnv_deg_mat[i].w);
         }
         if ((st = dev_upload(c, (noor_float4**)&S.tri, tri.data(), tri.size())) != NOOR_OK) return bail(st);
     }

@@ -150,9 +150,9 @@ struct DevScene {
     const uint4* __restrict__ wald0;
     const uint4* __restrict__ wald1;
     const uint4* __restrict__ wald2;
-    const float4* __restrict__ tri;      // watertight: v0, v1, v2 per triangle
+    const float4* __restrict__ tri;      // v0, v1, v2 per triangle; their w: caller's triangle id, instance (of a
+                                         // flat mesh's triangle), material type
     const uint4* __restrict__ attr;
-    const uint32_t* __restrict__ prim_ids;
     const float4* __restrict__ vert;
     const float4* __restrict__ nrm;
     const float2* __restrict__ uv;
@@ -170,6 +170,7 @@ struct DevScene {
     const float* __restrict__ dcdf;
     const noor_hosek* __restrict__ hosek;
     uint32_t wroot;          // reference of the root
+    uint32_t wroot_strict;   // and of the top level without flat meshes (wide_bvh.h); equal if there are none
     uint32_t gstack_lanes;   // lanes the global stack part is laid out for
     uint32_t n_area, n_point, n_spot, n_distant;
     int32_t num_lights;
@@ -476,6 +477,14 @@ __device__ __forceinline__ uint32_t box4_hit(const Ray& r, const WideNode& n, fl
     return mask & (meta >> 24);
 }
 
+// Per-triangle words beside the vertices (DevScene::tri).
+__device__ __forceinline__ uint32_t tri_word(const DevScene& S, uint32_t i, uint32_t k) {
+    return ldg(reinterpret_cast<const uint32_t*>(S.tri + 3 * (size_t)i + k) + 3);
+}
+__device__ __forceinline__ uint32_t tri_id(const DevScene& S, uint32_t i) { return tri_word(S, i, 0); }
+__device__ __forceinline__ uint32_t tri_inst(const DevScene& S, uint32_t i) { return tri_word(S, i, 1); }
+__device__ __forceinline__ uint32_t tri_type(const DevScene& S, uint32_t i) { return tri_word(S, i, 2); }
+
 struct Counters {
     uint32_t nodes, tris, tri2, inst;
 };
@@ -556,7 +565,7 @@ __device__ __forceinline__ bool tri_test(const DevScene& S, const Ray& r, uint32
                                          float& v, Counters& c) {
     if (STATS) c.tris++;
     const bool hit = (S.tri_test == NOOR_TRI_WALD) ? tri_wald(S, r, i, t, u, v, c) : tri_watertight(S, r, i, t, u, v);
-    if (ALPHA && hit && (ldg(S.wald2 + i).w & NOOR_MAT_ALPHA)) return alpha_pass(S, i, u, v);
+    if (ALPHA && hit && (tri_type(S, i) & NOOR_MAT_ALPHA)) return alpha_pass(S, i, u, v);
     return hit;
 }
 
@@ -699,7 +708,11 @@ struct Trav {
     Ray lray;
     uint32_t cur, ins;
     int sp;
-    bool hit, world;
+    // references that end lray's space: none in the world's; in an object's
+    // those with the TLAS bit; in a flat mesh's own, which only rays from
+    // wroot_strict enter, those of the top level itself
+    uint32_t leaves;
+    bool hit;
     Hit h;
 };
 
@@ -707,8 +720,10 @@ __device__ __forceinline__ void trav_begin(const DevScene& S, const Ray& r, Trav
     t.o = r.o;
     t.d = r.d;
     t.lray = r;
-    t.world = true;
-    t.cur = S.wroot;
+    t.leaves = 0u;
+    // zero, tiny, huge, infinite or NaN components: flat meshes through their instance
+    const float z = r.o.x * 0.0f + r.o.y * 0.0f + r.o.z * 0.0f;
+    t.cur = (r.pn & 16u) && z == 0.0f ? S.wroot : S.wroot_strict;
     t.ins = 0;
     t.sp = 0;
     t.hit = false;
@@ -744,7 +759,7 @@ __device__ __forceinline__ bool trav_steps(const DevScene& S, Trav& t, const Tra
     for (int step = 0; step < max_steps; ++step) {
         const uint32_t cur = t.cur;
         const uint32_t kind = (cur >> REF_KIND_SHIFT) & 3u;
-        if (kind == REF_INST || ((cur & REF_TLAS) && !t.world)) {
+        if (kind == REF_INST || (cur & t.leaves) != 0u) {
             f3 o = t.o, d = t.d;
             if (kind == REF_INST) {
                 t.ins = cur & REF_INDEX_MASK;
@@ -756,12 +771,13 @@ __device__ __forceinline__ bool trav_steps(const DevScene& S, Trav& t, const Tra
             t.lray.o = o;
             t.lray.d = d;
             ray_update_box(t.lray);
-            if (kind == REF_INST) ray_update_tri(t.lray);  // the top level holds no triangles
-            t.world = kind != REF_INST;
+            // the top level holds no triangles but those of flat meshes
+            if (kind == REF_INST || S.wroot != S.wroot_strict) ray_update_tri(t.lray);
+            t.leaves = 0u;  // an instance sets it with its root below
         }
         if (kind == REF_INNER) {
             if (STATS) c.nodes++;
-            const WideNode n = load_wnode(S, cur & REF_INDEX_MASK);
+            const WideNode n = load_wnode(S, cur & REF_NODE_MASK);
             float tn[4];
             const uint32_t m = box4_hit(t.lray, n, tn);
             if (m != 0u) {
@@ -793,12 +809,13 @@ __device__ __forceinline__ bool trav_steps(const DevScene& S, Trav& t, const Tra
                     t.hit = true;
                     return true;
                 }
-                const uint32_t key = ldg(S.prim_ids + ti);
+                const uint32_t key = tri_id(S, ti);
+                const uint32_t ins = (cur & REF_TLAS) ? tri_inst(S, ti) : t.ins;
                 bool take = false;
                 if (tt < t.lray.tmax) take = true;
                 else if (tt == t.lray.tmax) {
                     if (!t.hit) take = true;
-                    else if (key < t.h.key || (key == t.h.key && t.ins < t.h.inst)) take = true;
+                    else if (key < t.h.key || (key == t.h.key && ins < t.h.inst)) take = true;
                 }
                 if (take) {
                     t.hit = true;
@@ -808,7 +825,7 @@ __device__ __forceinline__ bool trav_steps(const DevScene& S, Trav& t, const Tra
                     t.h.v = v;
                     t.h.prim = ti;
                     t.h.key = key;
-                    t.h.inst = t.ins;
+                    t.h.inst = ins;
                     t.h.kind = 1;
                 }
             }
@@ -816,6 +833,7 @@ __device__ __forceinline__ bool trav_steps(const DevScene& S, Trav& t, const Tra
             if (t.cur != REF_EMPTY) continue;
         } else if (kind == REF_INST) {
             t.cur = ldg(S.inst_root + t.ins);
+            t.leaves = (t.cur & REF_TLAS) ? REF_LEAVES_FLAT : REF_TLAS;
             if (t.cur != REF_EMPTY) continue;
         } else {
             // light nodes are top-level references: lray is the world ray here
@@ -1276,7 +1294,7 @@ __device__ __forceinline__ void make_isect(const DevScene& S, const Ray& ray, co
         return;
     }
     I.tri = h.prim;
-    I.type = ldg(S.wald2 + h.prim).w;
+    I.type = tri_type(S, h.prim);
     const uint4 ai = ldg(S.attr + I.tri);
     I.mat = ai.w;
     if (I.type & M_EMITTER_ANY) {

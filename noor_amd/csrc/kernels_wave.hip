@@ -221,7 +221,7 @@ __device__ __forceinline__ void flush4(unsigned long long* dst, const Counters& 
 __device__ __forceinline__ int material_class(const DevScene& S, bool hit, const Hit& h) {
     if (!hit) return 0;
     if (h.kind == 2) return 1;
-    const uint32_t t = S.wald2[h.prim].w;
+    const uint32_t t = tri_type(S, h.prim);
     if (t & M_EMITTER_ANY) return 1;
     if (t == NOOR_MAT_DIFFUSE) return 2;
     if (t == NOOR_MAT_METAL) return 3;

@@ -123,14 +123,27 @@ class Builder {
     Builder(const noor_payload_view* P, WideBvh& W) : P_(P), W_(W) {}
 
     std::string run() {
-        W_.nodes.clear();
-        W_.inst_root.assign(P_->num_instances, REF_EMPTY);
-        const Child root = make_child(P_->bvh_root_node);
+        find_flat();
+        for (;;) {
+            W_.nodes.clear();
+            blas_.clear();
+            W_.inst_root.assign(P_->num_instances, REF_EMPTY);
+            W_.tri_inst.assign(flat_.empty() ? 0 : P_->num_triangles, REF_EMPTY);
+            direct_ = false;
+            W_.root = W_.root_strict = make_child(P_->bvh_root_node).ref;
+            if (err_.empty() && !flat_.empty()) {
+                direct_ = true;
+                W_.root = make_child(P_->bvh_root_node).ref;
+            }
+            if (!shared_tris_) break;
+            // two flat meshes hold one triangle, which then has no one instance
+            shared_tris_ = false;
+            flat_.clear();
+        }
         if (!err_.empty()) return err_;
-        W_.root = root.ref;
-        if (W_.nodes.size() >= REF_INDEX_MASK) return "too many wide BVH nodes";
+        if (W_.nodes.size() >= REF_NODE_MASK) return "too many wide BVH nodes";
         need_.assign(W_.nodes.size(), -1);
-        W_.stack_need = std::max<uint32_t>(1u, need(W_.root));
+        W_.stack_need = std::max<uint32_t>(1u, std::max(need(W_.root), need(W_.root_strict)));
         W_.qnodes.resize(W_.nodes.size());
         for (size_t i = 0; i < W_.nodes.size() && err_.empty(); ++i) err_ = quantize(W_.nodes[i], W_.qnodes[i]);
         return err_;
@@ -141,9 +154,39 @@ class Builder {
     WideBvh& W_;
     std::string err_;
     std::unordered_map<uint32_t, uint32_t> blas_;
+    std::unordered_map<uint32_t, uint32_t> flat_;  // BLAS root of a flat mesh -> its instance
+    bool direct_ = false;       // building the top level that refers to flat meshes directly
+    bool shared_tris_ = false;  // a triangle belongs to two flat meshes
     std::vector<int32_t> need_;
     std::vector<uint64_t> range_;
 
+    bool identity(uint32_t ins) const {
+        for (int r = 0; r < 3; ++r) {
+            const noor_float4 v = P_->world_to_object_row[r][ins];
+            const float e[4] = {v.x, v.y, v.z, v.w};
+            for (int c = 0; c < 4; ++c)
+                if (e[c] != (c == r ? 1.0f : 0.0f)) return false;
+        }
+        return true;
+    }
+    // The BLAS roots that exactly one instance places, by the identity.
+    void find_flat() {
+        std::unordered_map<uint32_t, uint32_t> uses;
+        std::vector<uint32_t> todo{P_->bvh_root_node};
+        while (!todo.empty()) {
+            const uint32_t i = todo.back();
+            todo.pop_back();
+            const BinKind k = kind(i);
+            if (k == B_INST) {
+                const uint32_t ins = flags(i) & NOOR_TRANS_MASK;
+                if (++uses[word(i)] == 1 && ins < P_->num_instances && identity(ins)) flat_[word(i)] = ins;
+            } else if (k == B_MLEAF || (k == B_INNER && tlas(i))) {
+                for (uint32_t j : expand(i)) todo.push_back(j);
+            }
+        }
+        for (const auto& u : uses)
+            if (u.second > 1) flat_.erase(u.first);
+    }
     uint32_t flags(uint32_t i) const { return P_->bvh_max_axis_count[i].w; }
     uint32_t word(uint32_t i) const { return P_->bvh_min_right_start[i].w; }
     BinKind kind(uint32_t i) const {
@@ -246,7 +289,7 @@ class Builder {
         }
     }
     // A wide node (or a small tree of them) over more than four children.
-    Child group(std::vector<Child> cs, bool is_tlas) {
+    Child group(std::vector<Child> cs, uint32_t level) {
         while (cs.size() > 4) {
             std::vector<Child> up;
             const size_t per = (cs.size() + 3) / 4;
@@ -261,7 +304,7 @@ class Builder {
                     }
                 const uint32_t idx = new_node();
                 fill(idx, part);
-                u.ref = (is_tlas ? REF_TLAS : 0u) | (REF_INNER << REF_KIND_SHIFT) | idx;
+                u.ref = level | (REF_INNER << REF_KIND_SHIFT) | idx;
                 up.push_back(u);
             }
             cs.swap(up);
@@ -274,7 +317,7 @@ class Builder {
                 u.lo[k] = std::min(u.lo[k], p.lo[k]);
                 u.hi[k] = std::max(u.hi[k], p.hi[k]);
             }
-        u.ref = (is_tlas ? REF_TLAS : 0u) | (REF_INNER << REF_KIND_SHIFT) | idx;
+        u.ref = level | (REF_INNER << REF_KIND_SHIFT) | idx;
         return u;
     }
 
@@ -286,12 +329,13 @@ class Builder {
             err_ = "instance points at a node that is not a BLAS root";
             return REF_EMPTY;
         }
-        const uint32_t r = make_child(b).ref;
+        const uint32_t r = make_child(b, flat_.count(b) ? (int64_t)flat_[b] : -1).ref;
         blas_[b] = r;
         return r;
     }
 
-    Child make_child(uint32_t i) {
+    // `flat`: the instance of the flat mesh node i belongs to, or -1.
+    Child make_child(uint32_t i, int64_t flat = -1) {
         Child c = box_of(i);
         if (!err_.empty()) return c;
         const uint32_t w = flags(i);
@@ -311,7 +355,7 @@ class Builder {
                 return c;
             }
             W_.inst_root[ins] = r;
-            c.ref = REF_TLAS | (REF_INST << REF_KIND_SHIFT) | ins;
+            c.ref = direct_ && r != REF_EMPTY && flat_.count(word(i)) ? r : REF_TLAS | (REF_INST << REF_KIND_SHIFT) | ins;
             return c;
         }
         case B_TLEAF: {
@@ -321,38 +365,45 @@ class Builder {
                 err_ = "more than 67108864 triangles";
                 return c;
             }
-            if (count <= REF_LEAF_MAX) {
-                c.ref = (REF_LEAF << REF_KIND_SHIFT) | ((count - 1) << REF_LEAF_COUNT_SHIFT) | start;
+            if (flat >= 0)
+                for (uint32_t t = start; t < start + count; ++t) {
+                    if (W_.tri_inst[t] != REF_EMPTY) shared_tris_ = true;
+                    W_.tri_inst[t] = (uint32_t)flat;
+                }
+            const uint32_t level = flat >= 0 ? REF_TLAS : 0u;
+            const uint32_t most = flat >= 0 ? REF_FLAT_LEAF_MAX : REF_LEAF_MAX;
+            if (count <= most) {
+                c.ref = level | (REF_LEAF << REF_KIND_SHIFT) | ((count - 1) << REF_LEAF_COUNT_SHIFT) | start;
                 return c;
             }
             std::vector<Child> parts;
-            for (uint32_t s = 0; s < count; s += REF_LEAF_MAX) {
+            for (uint32_t s = 0; s < count; s += most) {
                 Child p = c;
-                const uint32_t n = std::min(REF_LEAF_MAX, count - s);
-                p.ref = (REF_LEAF << REF_KIND_SHIFT) | ((n - 1) << REF_LEAF_COUNT_SHIFT) | (start + s);
+                const uint32_t n = std::min(most, count - s);
+                p.ref = level | (REF_LEAF << REF_KIND_SHIFT) | ((n - 1) << REF_LEAF_COUNT_SHIFT) | (start + s);
                 parts.push_back(p);
             }
-            return group(parts, false);
+            return group(parts, level);
         }
         case B_MLEAF:
         case B_INNER:
             break;
         }
-        if (small(i)) {
+        if (flat < 0 && small(i)) {
             uint32_t start = 0, count = 0;
             tri_range(i, start, count);
             c.ref = (REF_LEAF << REF_KIND_SHIFT) | ((count - 1) << REF_LEAF_COUNT_SHIFT) | start;
             return c;
         }
-        const bool is_tlas = tlas(i);
+        const uint32_t level = flat >= 0 ? REF_TLAS : (tlas(i) ? REF_TLAS | REF_TOP : 0u);
         std::vector<uint32_t> ch = expand(i);
         if (ch.size() > 4) {
             std::vector<Child> cs;
             for (uint32_t j : ch) {
-                Child cc = make_child(j);
+                Child cc = make_child(j, flat);
                 if (cc.ref != REF_EMPTY) cs.push_back(cc);
             }
-            return group(cs, is_tlas);
+            return group(cs, level);
         }
         // open the largest inner children while the node has room
         for (;;) {
@@ -374,11 +425,11 @@ class Builder {
         const uint32_t idx = new_node();
         std::vector<Child> cs;
         for (uint32_t j : ch) {
-            Child cc = make_child(j);
+            Child cc = make_child(j, flat);
             if (cc.ref != REF_EMPTY) cs.push_back(cc);
         }
         fill(idx, cs);
-        c.ref = (is_tlas ? REF_TLAS : 0u) | (REF_INNER << REF_KIND_SHIFT) | idx;
+        c.ref = level | (REF_INNER << REF_KIND_SHIFT) | idx;
         return c;
     }
 
@@ -392,7 +443,7 @@ class Builder {
             return ins < W_.inst_root.size() ? need(W_.inst_root[ins]) : 0u;
         }
         if (kind != REF_INNER) return 0;
-        const uint32_t idx = ref & REF_INDEX_MASK;
+        const uint32_t idx = ref & REF_NODE_MASK;
         if (need_[idx] >= 0) return (uint32_t)need_[idx];
         const WNode n = W_.nodes[idx];
         uint32_t k = 0, m = 0;
@@ -469,7 +520,7 @@ std::string check_wide_bvh(const noor_payload_view* P, const WideBvh& W) {
                 continue;
             }
             if (kind != REF_INNER) return "a BLAS references a TLAS node";
-            const uint32_t idx = ref & REF_INDEX_MASK;
+            const uint32_t idx = ref & REF_NODE_MASK;
             if (idx >= nn) return "wide node index out of range";
             const WNode& n = W.nodes[idx];
             for (int c = 0; c < 4; ++c) {
@@ -477,7 +528,7 @@ std::string check_wide_bvh(const noor_payload_view* P, const WideBvh& W) {
                 if (cr == REF_EMPTY) continue;
                 const uint32_t ck = (cr >> REF_KIND_SHIFT) & 3u;
                 if (ck == REF_INNER) {
-                    const WNode& m = W.nodes[cr & REF_INDEX_MASK];
+                    const WNode& m = W.nodes[cr & REF_NODE_MASK];
                     for (int d = 0; d < 4; ++d) {
                         if (m.ref[d] == REF_EMPTY) continue;
                         const float lo[3] = {m.lo[0][d], m.lo[1][d], m.lo[2][d]};
@@ -501,6 +552,37 @@ std::string check_wide_bvh(const noor_payload_view* P, const WideBvh& W) {
         std::sort(want.begin(), want.end());
         std::sort(got.begin(), got.end());
         if (want != got) return "a BLAS does not cover its triangles exactly once";
+    }
+    // both top levels reach every instance: as an instance, or (from `root`) a
+    // flat mesh's by its root
+    for (const uint32_t top : {W.root, W.root_strict}) {
+        std::vector<uint32_t> st{top}, got, want;
+        for (uint32_t i = 0; i < (uint32_t)W.inst_root.size(); ++i)
+            if (W.inst_root[i] != REF_EMPTY) want.push_back(W.inst_root[i]);
+        while (!st.empty()) {
+            const uint32_t ref = st.back();
+            st.pop_back();
+            const uint32_t kind = (ref >> REF_KIND_SHIFT) & 3u;
+            if (ref == REF_EMPTY || !(ref & REF_TLAS) || kind == REF_LIGHT) continue;
+            if (kind == REF_INST) {
+                if ((ref & REF_INDEX_MASK) >= W.inst_root.size()) return "instance out of range";
+                got.push_back(W.inst_root[ref & REF_INDEX_MASK]);
+            } else if (!(ref & REF_LEAVES_FLAT)) {
+                if (top == W.root_strict && W.root != W.root_strict) return "flat mesh in the strict top level";
+                got.push_back(ref);
+            } else {
+                if ((ref & REF_NODE_MASK) >= nn) return "wide node index out of range";
+                for (int c = 0; c < 4; ++c) st.push_back(W.nodes[ref & REF_NODE_MASK].ref[c]);
+            }
+        }
+        auto uniq = [](std::vector<uint32_t>& v) {
+            std::sort(v.begin(), v.end());
+            v.erase(std::unique(v.begin(), v.end()), v.end());
+            v.erase(std::remove(v.begin(), v.end(), REF_EMPTY), v.end());
+        };
+        uniq(got);
+        uniq(want);
+        if (got != want) return "a top level does not reach every instance";
     }
     if (W.stack_need < 1) return "stack bound";
     // compressed nodes: same references, decoded boxes around the exact ones

@@ -1,0 +1,75 @@
+"""Meshes placed by the identity (traversed with the world-space ray) beside transformed ones: structural check on the
+CPU, hit queries against the oracle and films of both renderers on the GPU."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from noor_amd import abi, scenes
+from noor_amd._lib import lib
+from noor_amd.renderer import Renderer, hits_to_numpy, rays_from_numpy
+from noor_amd.scene import Mesh, SceneBuilder, make_camera, make_options, make_spec, material
+from oracle.binding import OracleScene
+
+TURN = np.array([[0.0, 0.0, 1.0, 0.3], [0.0, 1.0, 0.0, 0.1], [-1.0, 0.0, 0.0, -0.2]])
+SHIFT = np.array([[1.0, 0.0, 0.0, 0.6], [0.0, 1.0, 0.0, 0.0], [0.0, 0.0, 1.0, 0.0]])
+EYE = np.eye(4)[:3]
+# (placements of the sphere, of the torus, triangles per leaf)
+LAYOUTS = {
+    "both_flat": ([EYE], [EYE], 2),
+    "flat_and_turned": ([EYE], [TURN], 2),
+    "two_identities": ([EYE, EYE], [SHIFT], 2),       # not flat: a hit has two candidate instances
+    "identity_and_shift": ([EYE, SHIFT], [EYE], 2),   # the sphere is not flat, the torus is
+    "leaves_of_8": ([EYE], [SHIFT], 8),               # flat leaves hold at most 4
+    "none_flat": ([TURN], [SHIFT], 2),
+}
+
+
+def _workload(layout):
+    spheres, tori, leaf = LAYOUTS[layout]
+    sb = SceneBuilder()
+    m = [sb.add_material(material(abi.MAT_DIFFUSE, diffuse=(0.6, 0.5, 0.4))),
+         sb.add_material(material(abi.MAT_METAL, eta=scenes.CU_ETA, k=scenes.CU_K, roughness=(0.2, 0.2)))]
+    sv, sf = scenes.icosphere(3)
+    tp, tt, tn, tu = scenes.torus(0.8, 0.25, 24, 12)
+    a = sb.add_mesh(Mesh(sv * 0.4, sf, normals=sv, material=m[0]))
+    b = sb.add_mesh(Mesh(tp, tt, normals=tn, uvs=tu, material=m[1]))
+    for M in spheres:
+        sb.add_instance(a, M)
+    for M in tori:
+        sb.add_instance(b, M)
+    sb.add_quad_light((-0.3, 1.5, -0.3), (0.6, 0, 0), (0, 0, 0.6), (5.0, 5.0, 5.0))
+    sb.set_env(scenes.env_map(64, 32, 5))
+    payload = sb.build(min_leaf=min(leaf, 2), max_leaf=leaf)
+    cam = make_camera((0.0, 1.2, 2.6), (0.0, 0.0, 0.0), (0, 1, 0), np.radians(50.0), 61, 47)
+    return scenes.Workload(layout, payload, cam, make_spec(payload, bounces=4), make_options(), None, 2)
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_wide_bvh_covers_flat_meshes(layout):
+    wl = _workload(layout)
+    assert lib().noor_wide_bvh_check(C.byref(wl.payload.view), None, None) == abi.OK
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_flat_meshes_match_oracle(layout):
+    wl = _workload(layout)
+    g = np.random.default_rng(41)
+    o = g.normal(size=(20000, 3))
+    o *= 3.0 / np.linalg.norm(o, axis=1, keepdims=True)
+    d = g.uniform(-0.7, 0.7, (20000, 3)) - o
+    rays = rays_from_numpy(o.astype(np.float32), d.astype(np.float32))
+    for tri in (abi.TRI_WATERTIGHT, abi.TRI_WALD):
+        wl.options.tri_test = tri
+        r, orc = Renderer.from_workload(wl), OracleScene.from_workload(wl)
+        hits = hits_to_numpy(r.trace(rays))
+        assert (hits[:, 6] > 0).sum() > 5000
+        np.testing.assert_array_equal(hits, hits_to_numpy(orc.trace(rays)[0]))
+        np.testing.assert_array_equal(hits_to_numpy(r.trace(rays, any_hit=True))[:, 6],
+                                      hits_to_numpy(orc.trace(rays, any_hit=True)[0])[:, 6])
+    r.render(2)
+    mega = r.film()
+    np.testing.assert_array_equal(mega, orc.render(1, 2)[0])
+    r.render_wavefront(2, frame=1)
+    np.testing.assert_array_equal(mega, r.film())
