@@ -239,8 +239,7 @@ struct Ray {
     f3 o, d, inv;
     float tmax;
     uint32_t pn;  // bit a set when d[a] <= 0 (the reference posneg); bit 3: box4_hit's fast form applies;
-                  // bit 4: no quotient of two components of d leaves the normal numbers
-    int kx, ky, kz;
+                  // bit 4: no quotient of two components of d leaves the normal numbers; bits 5-6: kz
     float Sx, Sy, Sz;
 };
 
@@ -285,30 +284,26 @@ __device__ __forceinline__ void ray_update_box(Ray& r) {
 
 // Triangle-test terms: Woop, Benthin & Wald, "Watertight Ray/Triangle
 // Intersection", JCGT 2(1), 2013 (axis permutation and shear).  Needs inv.
+// The permutation is a rotation, z the dominant axis; the paper's exchange of x
+// and y for a negative d[z] is left out: it only negates U, V, W and the
+// determinant together, which leaves the test, t, u and v as they are but for
+// the sign of a zero (tri_watertight restores it).
+__device__ __forceinline__ float perm_x(f3 v, bool z0, bool z1) { return z0 ? v.y : (z1 ? v.z : v.x); }
+__device__ __forceinline__ float perm_y(f3 v, bool z0, bool z1) { return z0 ? v.z : (z1 ? v.x : v.y); }
+__device__ __forceinline__ float perm_z(f3 v, bool z0, bool z1) { return z0 ? v.x : (z1 ? v.y : v.z); }
 __device__ __forceinline__ void ray_update_tri(Ray& r) {
     const float ax = fabsf(r.d.x), ay = fabsf(r.d.y), az = fabsf(r.d.z);
-    int kz = 0;
+    uint32_t kz = 0;
     float m = ax;
     if (ay > m) {
         kz = 1;
         m = ay;
     }
     if (az > m) kz = 2;
-    int kx = kz + 1;
-    if (kx == 3) kx = 0;
-    int ky = kx + 1;
-    if (ky == 3) ky = 0;
-    if (c3(r.d, kz) < 0.0f) {
-        const int t = kx;
-        kx = ky;
-        ky = t;
-    }
-    r.kx = kx;
-    r.ky = ky;
-    r.kz = kz;
-    const float dz = c3(r.d, kz);
-    r.Sz = c3(r.inv, kz);  // 1 / dz, already rounded once in inv
-    const float dx = c3(r.d, kx), dy = c3(r.d, ky);
+    r.pn = (r.pn & 31u) | (kz << 5);
+    const bool z0 = kz == 0, z1 = kz == 1;
+    const float dx = perm_x(r.d, z0, z1), dy = perm_y(r.d, z0, z1), dz = perm_z(r.d, z0, z1);
+    r.Sz = perm_z(r.inv, z0, z1);  // 1 / dz, already rounded once in inv
     if (r.pn & 16u) {
         r.Sx = div_by_rcp(dx, dz, r.Sz);
         r.Sy = div_by_rcp(dy, dz, r.Sz);
@@ -370,24 +365,23 @@ __device__ __forceinline__ Xf xf_from(const noor_transform& t) {
 // of a zero direction component.
 constexpr float BOX_SLACK = 1.00000095367431640625f;  // 1 + 2^-20
 
-// A compressed node (QNode in wide_bvh.h) as loaded: 56 of its 64 bytes.
+// A compressed node (QNode in wide_bvh.h) as loaded.
 struct WideNode {
-    uint4 a;  // org.xyz, meta
-    uint4 b;  // qlo.xyz, qhi.x
-    uint4 c;  // qhi.yz, ref0, ref1
-    uint2 d;  // ref2, ref3
-    __device__ __forceinline__ uint4 ref() const { return make_uint4(c.z, c.w, d.x, d.y); }
+    float4 a;  // org.xyz, scale.x
+    uint4 b;   // scale.yz, qlo.xy
+    uint4 c;   // qlo.z, qhi.xyz
+    uint4 ref;
 };
 __device__ __forceinline__ WideNode load_wnode(const DevScene& S, uint32_t idx) {
     const uint4* p = S.wbvh + (size_t)idx * 4;
     WideNode n;
-    n.a = ldg(p);
+    n.a = ldg(reinterpret_cast<const float4*>(p));
     n.b = ldg(p + 1);
     n.c = ldg(p + 2);
-    n.d = ldg(reinterpret_cast<const uint2*>(p + 3));
+    n.ref = ldg(p + 3);
     // the references are needed only when a child is entered, but loading
     // them then would add a second dependent fetch: issue them with the boxes
-    asm volatile("" ::"v"(n.d.x), "v"(n.d.y), "v"(n.c.z), "v"(n.c.w));
+    asm volatile("" ::"v"(n.ref.x), "v"(n.ref.y), "v"(n.ref.z), "v"(n.ref.w));
     return n;
 }
 // Plane c (byte c of q) of an axis with origin org and step s: the decode the
@@ -402,18 +396,14 @@ __device__ __forceinline__ float q_plane(float org, uint32_t q, int c, float s) 
 // (or subnormal) direction component: each plane is decoded as the builder
 // checked it (q_plane) and measured from the ray origin, the reference's
 // arithmetic (noor/cuda/bbox.cuh:62-80) including its infinities.
-__device__ __forceinline__ uint32_t box4_hit_exact(const Ray& r, const WideNode& n, float tn[4]) {
-    const float ox = __uint_as_float(n.a.x), oy = __uint_as_float(n.a.y), oz = __uint_as_float(n.a.z);
-    const uint32_t meta = n.a.w;
-    const float sx = __uint_as_float((meta & 0xFFu) << 23);
-    const float sy = __uint_as_float(((meta >> 8) & 0xFFu) << 23);
-    const float sz = __uint_as_float(((meta >> 16) & 0xFFu) << 23);
-    const uint32_t qlx = n.b.x, qly = n.b.y, qlz = n.b.z, qhx = n.b.w, qhy = n.c.x, qhz = n.c.y;
+__device__ __forceinline__ void box4_hit_exact(const Ray& r, const WideNode& n, float tn[4]) {
+    const float ox = n.a.x, oy = n.a.y, oz = n.a.z;
+    const float sx = fabsf(n.a.w), sy = fabsf(__uint_as_float(n.b.x)), sz = fabsf(__uint_as_float(n.b.y));
+    const uint32_t qlx = n.b.z, qly = n.b.w, qlz = n.c.x, qhx = n.c.y, qhy = n.c.z, qhz = n.c.w;
     const uint32_t nx = (r.pn & 1u) ? qhx : qlx, fx = (r.pn & 1u) ? qlx : qhx;
     const uint32_t ny = (r.pn & 2u) ? qhy : qly, fy = (r.pn & 2u) ? qly : qhy;
     const uint32_t nz = (r.pn & 4u) ? qhz : qlz, fz = (r.pn & 4u) ? qlz : qhz;
     const float tmaxs = r.tmax * BOX_SLACK;
-    uint32_t mask = 0;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         const float tx0 = (q_plane(ox, nx, c, sx) - r.o.x) * r.inv.x;
@@ -424,14 +414,12 @@ __device__ __forceinline__ uint32_t box4_hit_exact(const Ray& r, const WideNode&
         const float tz1 = (q_plane(oz, fz, c, sz) - r.o.z) * r.inv.z;
         const float t0 = fmaxf(fmaxf(tx0, ty0), tz0);
         const float t1 = fminf(fminf(tx1, ty1), tz1) * BOX_SLACK;
-        tn[c] = t0;
-        if (t0 <= t1 && t0 <= tmaxs && t1 >= 0.0f) mask |= 1u << c;
+        tn[c] = t0 <= t1 && t0 <= tmaxs && t1 >= 0.0f ? t0 : K_INF;
     }
-    return mask & (meta >> 24);
 }
 
-// Slab test of the four children of a compressed node.  Bit c of the result
-// is set when child c is entered; tn[c] is its entry distance.
+// Slab test of the four children of a compressed node: tn[c] is the entry
+// distance of child c, infinite if it is not entered (or slot c is empty).
 //
 // Per axis, A = (org - o) inv and B = s inv (exact: s is a power of two), and
 // the distance of plane q is one fused multiply-add, fma(q, B, A): two VALU
@@ -444,22 +432,19 @@ __device__ __forceinline__ uint32_t box4_hit_exact(const Ray& r, const WideNode&
 // the 2^-20 relative widening of exit distances and tmax; the absolute part by
 // W = 2^-22 max|A|, subtracted from entry and added to exit distances.  So a
 // box holding a point of the ray between 0 and tmax is always entered.
-__device__ __forceinline__ uint32_t box4_hit(const Ray& r, const WideNode& n, float tn[4]) {
-    if (!(r.pn & 8u)) return box4_hit_exact(r, n, tn);
-    const uint32_t meta = n.a.w;
-    const float sx = __uint_as_float((meta & 0xFFu) << 23);
-    const float sy = __uint_as_float(((meta >> 8) & 0xFFu) << 23);
-    const float sz = __uint_as_float(((meta >> 16) & 0xFFu) << 23);
-    const float Ax = (__uint_as_float(n.a.x) - r.o.x) * r.inv.x, Bx = sx * r.inv.x;
-    const float Ay = (__uint_as_float(n.a.y) - r.o.y) * r.inv.y, By = sy * r.inv.y;
-    const float Az = (__uint_as_float(n.a.z) - r.o.z) * r.inv.z, Bz = sz * r.inv.z;
+__device__ __forceinline__ void box4_hit(const Ray& r, const WideNode& n, float tn[4]) {
+    const float sy = __uint_as_float(n.b.x), sz = __uint_as_float(n.b.y);
+    const float Ax = (n.a.x - r.o.x) * r.inv.x, Bx = fabsf(n.a.w) * r.inv.x;
+    const float Ay = (n.a.y - r.o.y) * r.inv.y, By = fabsf(sy) * r.inv.y;
+    const float Az = (n.a.z - r.o.z) * r.inv.z, Bz = fabsf(sz) * r.inv.z;
     const float W = fmaxf(fmaxf(fabsf(Ax), fabsf(Ay)), fabsf(Az)) * 0x1p-22f;
-    const uint32_t qlx = n.b.x, qly = n.b.y, qlz = n.b.z, qhx = n.b.w, qhy = n.c.x, qhz = n.c.y;
-    const uint32_t nx = (r.pn & 1u) ? qhx : qlx, fx = (r.pn & 1u) ? qlx : qhx;
-    const uint32_t ny = (r.pn & 2u) ? qhy : qly, fy = (r.pn & 2u) ? qly : qhy;
-    const uint32_t nz = (r.pn & 4u) ? qhz : qlz, fz = (r.pn & 4u) ? qlz : qhz;
+    const uint32_t qlx = n.b.z, qly = n.b.w, qlz = n.c.x, qhx = n.c.y, qhy = n.c.z, qhz = n.c.w;
+    // finite reciprocals only: their signs are the direction's
+    const bool px = r.inv.x > 0.0f, py = r.inv.y > 0.0f, pz = r.inv.z > 0.0f;
+    const uint32_t nx = px ? qlx : qhx, fx = px ? qhx : qlx;
+    const uint32_t ny = py ? qly : qhy, fy = py ? qhy : qly;
+    const uint32_t nz = pz ? qlz : qhz, fz = pz ? qhz : qlz;
     const float tmaxs = r.tmax * BOX_SLACK;
-    uint32_t mask = 0;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         const float tx0 = __builtin_fmaf((float)((nx >> (8 * c)) & 0xFFu), Bx, Ax);
@@ -471,10 +456,8 @@ __device__ __forceinline__ uint32_t box4_hit(const Ray& r, const WideNode& n, fl
         // entered if t0 <= t1, t1 >= 0 and t0 <= tmaxs
         const float t0 = fmaxf(fmaxf(tx0, ty0), tz0) - W;
         const float t1 = __builtin_fmaf(fminf(fminf(tx1, ty1), tz1), BOX_SLACK, W);
-        tn[c] = t0;
-        if (fmaxf(t0, 0.0f) <= t1 && t0 <= tmaxs) mask |= 1u << c;
+        tn[c] = fmaxf(t0, 0.0f) <= t1 && t0 <= tmaxs ? t0 : K_INF;
     }
-    return mask & (meta >> 24);
 }
 
 // Per-triangle words beside the vertices (DevScene::tri).
@@ -527,13 +510,14 @@ __device__ __forceinline__ bool tri_watertight(const DevScene& S, const Ray& r, 
     const f3 A = sub3(f3{p0.x, p0.y, p0.z}, r.o);
     const f3 B = sub3(f3{p1.x, p1.y, p1.z}, r.o);
     const f3 C = sub3(f3{p2.x, p2.y, p2.z}, r.o);
-    const float Az0 = c3(A, r.kz), Bz0 = c3(B, r.kz), Cz0 = c3(C, r.kz);
-    const float Ax = c3(A, r.kx) - r.Sx * Az0;
-    const float Ay = c3(A, r.ky) - r.Sy * Az0;
-    const float Bx = c3(B, r.kx) - r.Sx * Bz0;
-    const float By = c3(B, r.ky) - r.Sy * Bz0;
-    const float Cx = c3(C, r.kx) - r.Sx * Cz0;
-    const float Cy = c3(C, r.ky) - r.Sy * Cz0;
+    const bool z0 = (r.pn & 0x60u) == 0u, z1 = (r.pn & 0x20u) != 0u;
+    const float Az0 = perm_z(A, z0, z1), Bz0 = perm_z(B, z0, z1), Cz0 = perm_z(C, z0, z1);
+    const float Ax = perm_x(A, z0, z1) - r.Sx * Az0;
+    const float Ay = perm_y(A, z0, z1) - r.Sy * Az0;
+    const float Bx = perm_x(B, z0, z1) - r.Sx * Bz0;
+    const float By = perm_y(B, z0, z1) - r.Sy * Bz0;
+    const float Cx = perm_x(C, z0, z1) - r.Sx * Cz0;
+    const float Cy = perm_y(C, z0, z1) - r.Sy * Cz0;
     float U = Cx * By - Cy * Bx;
     float V = Ax * Cy - Ay * Cx;
     float W = Bx * Ay - By * Ax;
@@ -553,6 +537,13 @@ __device__ __forceinline__ bool tri_watertight(const DevScene& S, const Ray& r, 
     to = t;
     uo = V * inv;
     vo = W * inv;
+    if (r.Sz < 0.0f) {
+        // x and y not exchanged: a zero edge function, or a sum that cancelled
+        // to zero, has the sign +0 either way while 1 / det has the other one
+        if (V == 0.0f) uo = -uo;
+        if (W == 0.0f) vo = -vo;
+        if (Tt == 0.0f && (U * Az != 0.0f || V * Bz != 0.0f)) to = -to;
+    }
     return true;
 }
 
@@ -633,7 +624,7 @@ __device__ __forceinline__ bool light_node_intersect(const DevScene& S, uint32_t
 
 struct Hit {
     float t, u, v;
-    uint32_t prim, key, inst, kind;
+    uint32_t prim, inst, kind;
 };
 
 // Per-lane traversal stack.  Entries [0, K) live in LDS, lane-interleaved
@@ -646,26 +637,29 @@ struct Hit {
 // one, and each wait for an LDS entry would also wait for the node loads in
 // flight.
 struct TravStack {
-    NOOR_LDS uint32_t* lds;
-    int lstride;
+    NOOR_LDS char* lds;
+    int shift;  // log2 of the bytes between a lane's entries
     int K;
     NOOR_GLOBAL uint32_t* glob;
     uint32_t gstride;
     int depth;
+    __device__ __forceinline__ void put_lds(int d, uint32_t v) const { *(NOOR_LDS uint32_t*)(lds + (d << shift)) = v; }
+    __device__ __forceinline__ uint32_t get_lds(int d) const { return *(NOOR_LDS uint32_t*)(lds + (d << shift)); }
     __device__ __forceinline__ void put(int d, uint32_t v) const {
-        if (d < K) lds[d * lstride] = v;
+        if (d < K) put_lds(d, v);
         else glob[(size_t)(d - K) * gstride] = v;
     }
     __device__ __forceinline__ uint32_t get(int d) const {
-        return d < K ? lds[d * lstride] : glob[(size_t)(d - K) * gstride];
+        return d < K ? get_lds(d) : glob[(size_t)(d - K) * gstride];
     }
 };
 // Stack of this lane whose entries beyond the LDS part live in `gstack`,
 // lane-interleaved over `glanes` lanes; the launch must use at most `glanes`.
+// blockDim.x is a power of two.
 __device__ __forceinline__ TravStack make_stack(const DevScene& S, uint32_t* smem, uint32_t* gstack, uint32_t glanes) {
     TravStack t;
-    t.lds = (NOOR_LDS uint32_t*)(smem + threadIdx.x);
-    t.lstride = (int)blockDim.x;
+    t.lds = (NOOR_LDS char*)(NOOR_LDS uint32_t*)(smem + threadIdx.x);
+    t.shift = 2 + __builtin_ctz(blockDim.x);
     t.K = S.stack_lds;
     t.glob = (NOOR_GLOBAL uint32_t*)(gstack + (blockIdx.x * blockDim.x + threadIdx.x));
     t.gstride = glanes;
@@ -677,9 +671,6 @@ __device__ __forceinline__ TravStack make_stack(const DevScene& S, uint32_t* sme
     return make_stack(S, smem, S.gstack, S.gstack_lanes);
 }
 
-__device__ __forceinline__ uint32_t ref_of(const uint4& r, int i) {
-    return i == 0 ? r.x : (i == 1 ? r.y : (i == 2 ? r.z : r.w));
-}
 __device__ __forceinline__ void cswap(float& a, float& b, uint32_t& ra, uint32_t& rb) {
     const bool s = b < a;
     const float ta = s ? b : a, tb = s ? a : b;
@@ -712,9 +703,23 @@ struct Trav {
     // those with the TLAS bit; in a flat mesh's own, which only rays from
     // wroot_strict enter, those of the top level itself
     uint32_t leaves;
-    bool hit;
-    Hit h;
+    // the hit so far: kind 0 none (an any-hit query sets 1), at distance
+    // lray.tmax; prim 0xFFFFFFFF for a light
+    float u, v;
+    uint32_t prim, inst, kind;
+    __device__ __forceinline__ bool hit() const { return kind != 0u; }
 };
+// The hit of a finished closest-hit traversal.
+__device__ __forceinline__ Hit trav_hit(const DevScene& S, const Trav& t) {
+    Hit h;
+    h.kind = t.kind;
+    h.t = t.kind ? t.lray.tmax : 0.0f;
+    h.u = t.u;
+    h.v = t.v;
+    h.prim = t.prim;
+    h.inst = t.inst;
+    return h;
+}
 
 __device__ __forceinline__ void trav_begin(const DevScene& S, const Ray& r, Trav& t) {
     t.o = r.o;
@@ -726,21 +731,29 @@ __device__ __forceinline__ void trav_begin(const DevScene& S, const Ray& r, Trav
     t.cur = (r.pn & 16u) && z == 0.0f ? S.wroot : S.wroot_strict;
     t.ins = 0;
     t.sp = 0;
-    t.hit = false;
-    t.h.kind = 0;
-    t.h.prim = 0xFFFFFFFFu;
-    t.h.key = 0xFFFFFFFFu;
-    t.h.inst = 0xFFFFFFFFu;
-    t.h.t = 0.0f;
-    t.h.u = t.h.v = 0.0f;
+    t.kind = 0;
+    t.prim = 0xFFFFFFFFu;
+    t.inst = 0xFFFFFFFFu;
+    t.u = t.v = 0.0f;
 }
 
+// The traversal kernels are bound by the VALU instructions of a step, of which
+// the inner-node block is most: about 140 with the scales stored as floats, slot
+// signs instead of a mask, children sorted as they are tested, stack entries at
+// shifted LDS addresses and one wave-wide check for the LDS part.  Before, with
+// byte exponents, a hit mask, a multiply per stack access and a check per entry,
+// about 210: the 1080p terrain film took 42.2 instead of 40.3 ms, the 1M-triangle
+// film 27.1 instead of 26.3.
+//
 // One step of a traversal visits one inner node, tests ONE triangle of a leaf
 // (a leaf with triangles left stays the current reference, its start advanced
 // and its count decremented), enters one instance or tests one light.  Lanes
 // of a wave step in lockstep, so a wave pays for the union of the kinds its
 // lanes visit in a step: testing a whole leaf per step would make every step
 // with a leaf lane cost as many triangle tests as the wave's largest leaf.
+// Letting leaf lanes wait until 4, 8, 16 or 24 of a wave's have one costs as
+// much as it gains at 4 and 8 (terrain film 41.0, 41.3 against 41.1 ms) and more
+// beyond (43.1, 45.5); waiting instance lanes cost 7%.
 // The ray of the level is rebuilt in one place for both transitions that need
 // it: entering an instance (object space) and popping back to the top level
 // (world space); a pop straight into another instance builds only the
@@ -751,12 +764,13 @@ __device__ __forceinline__ uint32_t leaf_next(uint32_t cur) {
 
 //
 // KIND: a closest-hit query, an any-hit one (ends at the first triangle or light
-// it finds, t.hit), or the lane's choice in `any`.
+// it finds, t.hit()), or the lane's choice in `any`.
 enum : int { TRAV_CLOSEST, TRAV_ANY, TRAV_MIXED };
 template <bool STATS, bool ALPHA, int KIND>
 __device__ __forceinline__ bool trav_steps(const DevScene& S, Trav& t, const TravStack& st, Counters& c,
                                            bool& overflow, int max_steps, bool any = KIND == TRAV_ANY) {
-    for (int step = 0; step < max_steps; ++step) {
+    bool done = false;
+    for (int step = 0; step < max_steps && !done; ++step) {
         const uint32_t cur = t.cur;
         const uint32_t kind = (cur >> REF_KIND_SHIFT) & 3u;
         if (kind == REF_INST || (cur & t.leaves) != 0u) {
@@ -775,91 +789,104 @@ __device__ __forceinline__ bool trav_steps(const DevScene& S, Trav& t, const Tra
             if (kind == REF_INST || S.wroot != S.wroot_strict) ray_update_tri(t.lray);
             t.leaves = 0u;  // an instance sets it with its root below
         }
+        uint32_t next = REF_EMPTY;  // REF_EMPTY: take the next entry off the stack
         if (kind == REF_INNER) {
             if (STATS) c.nodes++;
             const WideNode n = load_wnode(S, cur & REF_NODE_MASK);
-            float tn[4];
-            const uint32_t m = box4_hit(t.lray, n, tn);
-            if (m != 0u) {
-                float d0 = (m & 1u) ? tn[0] : K_INF, d1 = (m & 2u) ? tn[1] : K_INF;
-                float d2 = (m & 4u) ? tn[2] : K_INF, d3 = (m & 8u) ? tn[3] : K_INF;
-                const uint4 rf = n.ref();
-                uint32_t r0 = rf.x, r1 = rf.y, r2 = rf.z, r3 = rf.w;
-                cswap(d0, d1, r0, r1);
-                cswap(d2, d3, r2, r3);
-                cswap(d0, d2, r0, r2);
-                cswap(d1, d3, r1, r3);
-                cswap(d1, d2, r1, r2);
-                const int k = __popc(m);
-                if (t.sp + k - 1 > st.depth) {
+            float d[4];
+            box4_hit(t.lray, n, d);
+            if (__ballot(!(t.lray.pn & 8u)) != 0ull) {
+                if (!(t.lray.pn & 8u)) box4_hit_exact(t.lray, n, d);
+            }
+            float d0 = d[0], d1 = __uint_as_float(n.b.y) > 0.0f ? d[1] : K_INF;
+            float d2 = __uint_as_float(n.b.x) > 0.0f ? d[2] : K_INF, d3 = n.a.w > 0.0f ? d[3] : K_INF;
+            uint32_t r0 = n.ref.x, r1 = n.ref.y, r2 = n.ref.z, r3 = n.ref.w;
+            cswap(d0, d1, r0, r1);
+            cswap(d2, d3, r2, r3);
+            cswap(d0, d2, r0, r2);
+            cswap(d1, d3, r1, r3);
+            cswap(d1, d2, r1, r2);
+            if (d0 < K_INF) next = r0;
+            if (__ballot(t.sp + 3 > st.K) == 0ull) {
+                // the usual case: all of the wave's entries fit in LDS
+                if (d3 < K_INF) st.put_lds(t.sp++, r3);
+                if (d2 < K_INF) st.put_lds(t.sp++, r2);
+                if (d1 < K_INF) st.put_lds(t.sp++, r1);
+            } else {
+                const int k = (d1 < K_INF ? 1 : 0) + (d2 < K_INF ? 1 : 0) + (d3 < K_INF ? 1 : 0);
+                if (t.sp + k > st.depth) {
                     overflow = true;
-                    return true;
+                    t.sp = 0;
+                    next = REF_EMPTY;
+                } else {
+                    if (k > 2) st.put(t.sp++, r3);
+                    if (k > 1) st.put(t.sp++, r2);
+                    if (k > 0) st.put(t.sp++, r1);
                 }
-                if (k > 3) st.put(t.sp++, r3);
-                if (k > 2) st.put(t.sp++, r2);
-                if (k > 1) st.put(t.sp++, r1);
-                t.cur = r0;
-                continue;
             }
         } else if (kind == REF_LEAF) {
             const uint32_t ti = cur & REF_LEAF_START_MASK;
+            next = leaf_next(cur);
             float tt, u, v;
             if (tri_test<STATS, ALPHA>(S, t.lray, ti, tt, u, v, c)) {
                 if (KIND != TRAV_CLOSEST && any) {
-                    t.hit = true;
-                    return true;
-                }
-                const uint32_t key = tri_id(S, ti);
-                const uint32_t ins = (cur & REF_TLAS) ? tri_inst(S, ti) : t.ins;
-                bool take = false;
-                if (tt < t.lray.tmax) take = true;
-                else if (tt == t.lray.tmax) {
-                    if (!t.hit) take = true;
-                    else if (key < t.h.key || (key == t.h.key && ins < t.h.inst)) take = true;
-                }
-                if (take) {
-                    t.hit = true;
-                    t.lray.tmax = tt;
-                    t.h.t = tt;
-                    t.h.u = u;
-                    t.h.v = v;
-                    t.h.prim = ti;
-                    t.h.key = key;
-                    t.h.inst = ins;
-                    t.h.kind = 1;
+                    t.kind = 1;
+                    t.sp = 0;
+                    next = REF_EMPTY;
+                } else {
+                    const uint32_t ins = (cur & REF_TLAS) ? tri_inst(S, ti) : t.ins;
+                    bool take = tt < t.lray.tmax;
+                    if (tt == t.lray.tmax) {
+                        // a light loses ties; two triangles are ordered by caller's id, then instance
+                        take = t.prim == 0xFFFFFFFFu;
+                        if (!take) {
+                            const uint32_t key = tri_id(S, ti), old = tri_id(S, t.prim);
+                            take = key < old || (key == old && ins < t.inst);
+                        }
+                    }
+                    if (take) {
+                        t.lray.tmax = tt;
+                        t.u = u;
+                        t.v = v;
+                        t.prim = ti;
+                        t.inst = ins;
+                        t.kind = 1;
+                    }
                 }
             }
-            t.cur = leaf_next(cur);
-            if (t.cur != REF_EMPTY) continue;
         } else if (kind == REF_INST) {
-            t.cur = ldg(S.inst_root + t.ins);
-            t.leaves = (t.cur & REF_TLAS) ? REF_LEAVES_FLAT : REF_TLAS;
-            if (t.cur != REF_EMPTY) continue;
-        } else {
+            next = ldg(S.inst_root + t.ins);
+            t.leaves = (next & REF_TLAS) ? REF_LEAVES_FLAT : REF_TLAS;
+        } else if (cur != REF_EMPTY) {  // (an empty scene's root)
             // light nodes are top-level references: lray is the world ray here
             const uint32_t li = cur & REF_INDEX_MASK;
             Ray tr = t.lray;
             const bool lh = light_node_intersect(S, li, tr);
             if (KIND != TRAV_CLOSEST && any) {
                 if (lh) {
-                    t.hit = true;
-                    return true;
+                    t.kind = 1;
+                    t.sp = 0;
                 }
             } else if (lh && tr.tmax < t.lray.tmax) {
                 t.lray.tmax = tr.tmax;
-                t.hit = true;
-                t.h.t = tr.tmax;
-                t.h.kind = 2;
-                t.h.inst = li;
-                t.h.key = 0xFFFFFFFFu;
-                t.h.prim = 0xFFFFFFFFu;
-                t.h.u = t.h.v = 0.0f;
+                t.kind = 2;
+                t.inst = li;
+                t.prim = 0xFFFFFFFFu;
+                t.u = t.v = 0.0f;
             }
         }
-        if (t.sp == 0) return true;
-        t.cur = st.get(--t.sp);
+        if (next == REF_EMPTY) {
+            if (t.sp == 0) {
+                done = true;
+            } else {
+                --t.sp;
+                if (__ballot(t.sp >= st.K) == 0ull) next = st.get_lds(t.sp);
+                else next = st.get(t.sp);
+            }
+        }
+        t.cur = next;
     }
-    return false;
+    return done;
 }
 
 template <bool STATS, bool ALPHA = false>
@@ -870,8 +897,8 @@ __device__ __forceinline__ bool bvh_closest(const DevScene& S, Ray& ray, Hit& h,
     while (!trav_steps<STATS, ALPHA, TRAV_CLOSEST>(S, t, st, c, overflow, 1 << 30)) {
     }
     ray.tmax = t.lray.tmax;
-    h = t.h;
-    return t.hit;
+    h = trav_hit(S, t);
+    return t.hit();
 }
 
 template <bool STATS, bool ALPHA = false>
@@ -881,7 +908,7 @@ __device__ __forceinline__ bool bvh_any(const DevScene& S, const Ray& ray, const
     trav_begin(S, ray, t);
     while (!trav_steps<STATS, ALPHA, TRAV_ANY>(S, t, st, c, overflow, 1 << 30)) {
     }
-    return t.hit;
+    return t.hit();
 }
 
 // ---------------------------------------------------------------------------------------------

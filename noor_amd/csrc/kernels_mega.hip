@@ -186,7 +186,7 @@ __global__ __launch_bounds__(64) void k_trace(const DevScene* __restrict__ Sp, c
                 out.inst = h.inst;
                 if (h.kind == 1) {
                     out.prim = h.prim;
-                    out.prim_id = h.key;
+                    out.prim_id = tri_id(S, h.prim);
                 }
             }
         }

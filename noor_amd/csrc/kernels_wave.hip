@@ -419,8 +419,11 @@ __device__ __forceinline__ uint32_t refill(uint32_t* work, uint32_t count, bool 
     return !have && valid ? idx : 0xFFFFFFFFu;
 }
 
-// Held to 80 VGPRs (six waves per SIMD, a few spilled registers): measured 6%
-// faster than 84 VGPRs at five waves.
+// 79 VGPRs, six waves per SIMD, no spills: the traversal issues a VALU
+// instruction in nearly every slot (SQ_ACTIVE_INST_VALU at 97% of the SIMDs'
+// issue slots on the 1080p terrain), so its time follows the instructions of a
+// step.  At five waves the terrain film's k_extend takes 20.5 instead of 19.1
+// ms, at seven (spills) 25.5.
 template <bool STATS, bool ALPHA>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_extend(
     const DevScene* __restrict__ Sp, WavePool B, int cur, DevStats* stats) {
@@ -433,32 +436,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
     Counters cnt{0, 0, 0, 0};
     bool overflow = false, have = false;
     Claim claim{0u, 0u, count == 0u};
-    uint32_t ext = 0, nhit = 0;  // rays this lane started, and (STATS) how many hit
-    uint32_t p = 0, qi = 0;
+    uint32_t ext = 0, nhit = 0;  // rays this wave started, and (STATS) how many this lane's hit
+    uint32_t qi = 0;
     Trav t;
     for (;;) {
         const uint32_t idx = refill<2>(&ctl->work_extend.v, count, have, claim);
+        ext += (uint32_t)__popcll(__ballot(idx != 0xFFFFFFFFu));
         if (idx != 0xFFFFFFFFu) {
-            p = q[idx];
             const float4 o = B.qo[cur][idx], d = B.qd[cur][idx];
             qi = (idx << 3) | (o.w != 0.0f ? 4u : 0u);
             trav_begin(S, mkray(f3{o.x, o.y, o.z}, f3{d.x, d.y, d.z}, K_INF), t);
             have = true;
-            ++ext;
         }
         if (__ballot(have) == 0ull) break;
         if (have && trav_steps<STATS, ALPHA, TRAV_CLOSEST>(S, t, st, cnt, overflow, B.steps)) {
-            B.hit[2 * (size_t)p] = make_uint4(__float_as_uint(t.h.t), __float_as_uint(t.h.u), __float_as_uint(t.h.v),
-                                              t.h.prim);
-            B.hit[2 * (size_t)p + 1] = make_uint4(t.h.inst, (t.hit ? t.h.kind : 0u) | qi, 0u, 0u);
-            B.cls[p] = (uint32_t)material_class(S, t.hit, t.h);
-            if (STATS && t.hit) ++nhit;
+            const Hit h = trav_hit(S, t);
+            const uint32_t p = q[qi >> 3];
+            B.hit[2 * (size_t)p] = make_uint4(__float_as_uint(h.t), __float_as_uint(h.u), __float_as_uint(h.v), h.prim);
+            B.hit[2 * (size_t)p + 1] = make_uint4(h.inst, h.kind | qi, 0u, 0u);
+            B.cls[p] = (uint32_t)material_class(S, t.hit(), h);
+            if (STATS && t.hit()) ++nhit;
             have = false;
         }
     }
-    unsigned long long e = ext;
-    for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);  // 64-bit wave sum
-    if (lane_id() == 0 && e) atomicAdd(&stats->slot[stat_slot()].extension_rays, e);
+    if (lane_id() == 0 && ext) atomicAdd(&stats->slot[stat_slot()].extension_rays, (unsigned long long)ext);
     if (STATS) {
         flush4(stats->ext, cnt);
         unsigned long long h = nhit;
@@ -575,7 +576,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TEX ? 2 : 4
         h.prim = __float_as_uint(hh.w);
         h.inst = h2.x;
         h.kind = h2.y & 3u;
-        h.key = 0;
         const bool hit = h.kind != 0;
         if (hit) ray.tmax = h.t;
         Nee nee;
@@ -678,9 +678,12 @@ __global__ __launch_bounds__(1024) void k_collect_free(WavePool B, int cur) {
 }
 
 // MIS: a task may hold a second, BSDF-sampled shadow ray (separate
-// instantiation, so the kernel without MIS keeps its registers)
+// instantiation, so the kernel without MIS keeps its registers).  Held to six
+// waves per SIMD: 91 VGPRs at five take 7.9 instead of 7.6 ms of the 1080p
+// terrain film, 2.3 instead of 2.4 ms of a 200k-pixel film with MIS; seven gain
+// nothing.
 template <bool STATS, bool ALPHA, bool MIS>
-__global__ void k_shadow(const DevScene* __restrict__ Sp, WavePool B, DevStats* stats) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_shadow(const DevScene* __restrict__ Sp, WavePool B, DevStats* stats) {
     const DevScene& S = *Sp;
     extern __shared__ uint32_t smem[];
     WaveCtl* ctl = B.ctl;
@@ -710,7 +713,7 @@ __global__ void k_shadow(const DevScene* __restrict__ Sp, WavePool B, DevStats* 
         if (have && trav_steps<STATS, ALPHA, TRAV_ANY>(S, t, st, cnt, overflow, B.steps)) {
             const bool nb = MIS && B.nee_b[p].w != 0.0f;
             if (!second && nb) {
-                occ_a = t.hit;
+                occ_a = t.hit();
                 second = true;
                 const float4 o = B.sh2_o[p], d = B.sh2_d[p];
                 trav_begin(S, mkray(f3{o.x, o.y, o.z}, f3{d.x, d.y, d.z}, o.w), t);
@@ -728,8 +731,8 @@ __global__ void k_shadow(const DevScene* __restrict__ Sp, WavePool B, DevStats* 
                 const float4 b = B.nee_b[p];
                 nee.b = f3{b.x, b.y, b.z};
             }
-            const bool oa = nee.na ? (second && nb ? occ_a : t.hit) : false;
-            const bool ob = nb ? t.hit : false;
+            const bool oa = nee.na ? (second && nb ? occ_a : t.hit()) : false;
+            const bool ob = nb ? t.hit() : false;
             PathState ps;
             const float4 L = B.Lb[2 * (size_t)p];
             ps.L = f3{L.x, L.y, L.z};

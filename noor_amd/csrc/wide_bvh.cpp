@@ -34,7 +34,7 @@ double q_exact(float org, uint32_t q, float s) { return (double)org + (double)q 
 
 // Encodes one axis of one node: the smallest power-of-two step for which every
 // slot's rounded-out planes fit in 8 bits.  Returns false if none does.
-bool quantize_axis(const WNode& n, int a, uint32_t valid, float& org, uint32_t& ebyte, uint32_t& qlo, uint32_t& qhi) {
+bool quantize_axis(const WNode& n, int a, uint32_t valid, float& org, float& scale, uint32_t& qlo, uint32_t& qhi) {
     float lo = std::numeric_limits<float>::infinity(), hi = -std::numeric_limits<float>::infinity();
     for (int c = 0; c < 4; ++c)
         if (valid & (1u << c)) {
@@ -78,7 +78,7 @@ bool quantize_axis(const WNode& n, int a, uint32_t valid, float& org, uint32_t& 
             H |= (uint32_t)r << (8 * c);
         }
         if (ok) {
-            ebyte = (uint32_t)(k + 127);
+            scale = s;
             qlo = L;
             qhi = H;
             return true;
@@ -94,12 +94,11 @@ std::string quantize(const WNode& n, QNode& q) {
         q.ref[c] = n.ref[c];
         if (n.ref[c] != REF_EMPTY) valid |= 1u << c;
     }
-    q.meta = valid << 24;
+    if (!valid || (valid & (valid + 1))) return "a node's children do not fill its slots from 0 on";
     for (int a = 0; a < 3; ++a) {
-        uint32_t e = 0;
-        if (!quantize_axis(n, a, valid, q.org[a], e, q.qlo[a], q.qhi[a]))
+        if (!quantize_axis(n, a, valid, q.org[a], q.scale[a], q.qlo[a], q.qhi[a]))
             return "a node box cannot be quantised (non-finite or too large a range)";
-        q.meta |= e << (8 * a);
+        if (!(valid & (8u >> a))) q.scale[a] = -q.scale[a];
     }
     return std::string();
 }
@@ -290,6 +289,11 @@ class Builder {
     }
     // A wide node (or a small tree of them) over more than four children.
     Child group(std::vector<Child> cs, uint32_t level) {
+        if (cs.empty()) {
+            Child none{};
+            none.ref = REF_EMPTY;
+            return none;
+        }
         while (cs.size() > 4) {
             std::vector<Child> up;
             const size_t per = (cs.size() + 3) / 4;
@@ -311,7 +315,7 @@ class Builder {
         }
         const uint32_t idx = new_node();
         fill(idx, cs);
-        Child u = cs.empty() ? Child{} : cs[0];
+        Child u = cs[0];
         for (const Child& p : cs)
             for (int k = 0; k < 3; ++k) {
                 u.lo[k] = std::min(u.lo[k], p.lo[k]);
@@ -427,6 +431,10 @@ class Builder {
         for (uint32_t j : ch) {
             Child cc = make_child(j, flat);
             if (cc.ref != REF_EMPTY) cs.push_back(cc);
+        }
+        if (cs.empty()) {  // only empty leaves below: no node (none was added after it)
+            W_.nodes.pop_back();
+            return c;
         }
         fill(idx, cs);
         c.ref = level | (REF_INNER << REF_KIND_SHIFT) | idx;
@@ -592,11 +600,11 @@ std::string check_wide_bvh(const noor_payload_view* P, const WideBvh& W) {
         const QNode& q = W.qnodes[i];
         for (int c = 0; c < 4; ++c) {
             if (q.ref[c] != n.ref[c]) return "compressed node reference";
-            const bool valid = ((q.meta >> 24) >> c) & 1u;
-            if (valid != (n.ref[c] != REF_EMPTY)) return "compressed node slot mask";
+            const bool valid = c == 0 || !std::signbit(q.scale[3 - c]);
+            if (valid != (n.ref[c] != REF_EMPTY)) return "compressed node slot signs";
             if (!valid) continue;
             for (int a = 0; a < 3; ++a) {
-                const float s = std::ldexp(1.0f, (int)((q.meta >> (8 * a)) & 0xFFu) - 127);
+                const float s = std::fabs(q.scale[a]);
                 const uint32_t ql = (q.qlo[a] >> (8 * c)) & 0xFFu, qh = (q.qhi[a] >> (8 * c)) & 0xFFu;
                 const float lo = q_decode(q.org[a], ql, s);
                 const float hi = q_decode(q.org[a], qh, s);

@@ -65,24 +65,24 @@ struct alignas(128) WNode {
 };
 static_assert(sizeof(WNode) == 128, "WNode is one 128-byte line");
 
-// Device form, 64 bytes (56 read per visit): the four child boxes quantised
-// to 8 bits per plane on a grid local to the node (as in Ylitie, Karras &
-// Laine, "Efficient Incoherent Ray Traversal on GPUs Through Compressed Wide
-// BVHs", HPG 2017).  On axis a a plane decodes to
-//     org[a] + (float)q * 2^(e[a] - 127)        (binary32, no contraction)
-// with e[a] = byte a of `meta`.  The encoder rounds lower planes down and upper
-// planes up and checks the decoded values, so every decoded box contains its
-// child's exact box; with the conservative slab test the traversal therefore
-// returns the same hits as over the exact boxes.  Byte 3 of `meta` has bit c
-// set when slot c holds a child.  Words: [org.xyz, meta] [qlo.xyz, qhi.x]
-// [qhi.yz, ref0, ref1] [ref2, ref3, pad, pad]; slot c is byte c of each q word.
+// Device form, 64 bytes: the four child boxes quantised to 8 bits per plane on
+// a grid local to the node (as in Ylitie, Karras & Laine, "Efficient Incoherent
+// Ray Traversal on GPUs Through Compressed Wide BVHs", HPG 2017).  On axis a a
+// plane decodes to
+//     org[a] + (float)q * |scale[a]|            (binary32, no contraction)
+// with |scale[a]| a power of two.  The encoder rounds lower planes down and
+// upper planes up and checks the decoded values, so every decoded box contains
+// its child's exact box; with the conservative slab test the traversal
+// therefore returns the same hits as over the exact boxes.  The children fill
+// the slots from 0 on; slot 0 is never empty, and the signs of the scales say
+// which others are: scale[2] negative for slot 1, scale[1] for slot 2, scale[0]
+// for slot 3.  Slot c is byte c of each q word.
 struct alignas(64) QNode {
     float org[3];
-    uint32_t meta;
+    float scale[3];
     uint32_t qlo[3];
     uint32_t qhi[3];
     uint32_t ref[4];
-    uint32_t pad[2];
 };
 static_assert(sizeof(QNode) == 64, "QNode is 64 bytes");
 
