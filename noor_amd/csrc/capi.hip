@@ -404,30 +404,45 @@ noor_status noor_create(const noor_payload_view* P, const noor_hosek* hosek, con
     if ((st = dev_upload(c, (noor_uint4**)&S.wald0, P->wald_ax_nu_nv_nd, nt)) != NOOR_OK) return bail(st);
     if ((st = dev_upload(c, (noor_uint4**)&S.wald1, P->wald_bnu_bnv_au_av, nt)) != NOOR_OK) return bail(st);
     if ((st = dev_upload(c, (noor_uint4**)&S.wald2, P->wald_cnu_cnv_deg_mat, nt)) != NOOR_OK) return bail(st);
-    if ((st = dev_upload(c, (noor_uint4**)&S.attr, P->attribute_indices, nt)) != NOOR_OK) return bail(st);
     {
-        // the three vertices of each triangle in leaf order, with what a hit needs of it in their fourth words
-        std::vector<noor_float4> tri((size_t)3 * (nt ? nt : 1));
-        auto word = [](uint32_t u) {
-            float f;
-            std::memcpy(&f, &u, 4);
-            return f;
-        };
-        for (uint32_t i = 0; i < nt; ++i) {
-            const noor_uint4 a = P->attribute_indices[i];
-            noor_float4* t = &tri[3 * (size_t)i];
-            t[0] = P->vertices[a.x];
-            t[1] = P->vertices[a.y];
-            t[2] = P->vertices[a.z];
-            t[0].w = word(P->prim_ids ? P->prim_ids[i] : i);
-            t[1].w = word(flat_inst.empty() ? 0u : flat_inst[i]);
-            t[2].w = word(P->wald_cnu_cnv_deg_mat[i].w);
+        // per-triangle records, gathered on the device from the payload's vertex arrays, which are not kept
+        noor_uint4* attr = nullptr;
+        noor_float4 *vert = nullptr, *nrm = nullptr;
+        noor_float2* uv = nullptr;
+        uint32_t *ids = nullptr, *inst = nullptr;
+        std::vector<uint32_t> count_up;
+        if (!P->prim_ids) {
+            count_up.resize(nt);
+            for (uint32_t i = 0; i < nt; ++i) count_up[i] = i;
         }
-        if ((st = dev_upload(c, (noor_float4**)&S.tri, tri.data(), tri.size())) != NOOR_OK) return bail(st);
+        const size_t kept = c->allocs.size();
+        if ((st = dev_upload(c, &attr, P->attribute_indices, nt)) != NOOR_OK) return bail(st);
+        if ((st = dev_upload(c, &vert, P->vertices, P->num_vertices)) != NOOR_OK) return bail(st);
+        if ((st = dev_upload(c, &nrm, P->normals, P->num_vertices)) != NOOR_OK) return bail(st);
+        if ((st = dev_upload(c, &uv, P->uvs, P->num_vertices)) != NOOR_OK) return bail(st);
+        if ((st = dev_upload(c, &ids, P->prim_ids ? P->prim_ids : count_up.data(), nt)) != NOOR_OK) return bail(st);
+        if (!flat_inst.empty() && (st = dev_upload(c, &inst, flat_inst.data(), nt)) != NOOR_OK) return bail(st);
+        const std::vector<void*> temporary(c->allocs.begin() + kept, c->allocs.end());
+        c->allocs.resize(kept);
+        void *tri = nullptr, *shade = nullptr;
+        hipError_t e = hipMalloc(&tri, sizeof(float4) * 3 * (size_t)std::max(nt, 1u));
+        if (e == hipSuccess) {
+            c->allocs.push_back(tri);
+            e = hipMalloc(&shade, sizeof(float4) * 4 * (size_t)std::max(nt, 1u));
+        }
+        if (e == hipSuccess) {
+            c->allocs.push_back(shade);
+            S.tri = (const float4*)tri;
+            S.shade = (const float4*)shade;
+            e = noor::launch_tri_records(*c, (const uint4*)attr, (const float4*)vert, (const float4*)nrm,
+                                         (const float2*)uv, ids, inst);
+        }
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        for (void* p : temporary) hipFree(p);
+        if (e != hipSuccess)
+            return bail(fail(c, e == hipErrorOutOfMemory ? NOOR_ERR_OUT_OF_MEMORY : NOOR_ERR_HIP,
+                             std::string("triangle records: ") + hipGetErrorString(e)));
     }
-    if ((st = dev_upload(c, (noor_float4**)&S.vert, P->vertices, P->num_vertices)) != NOOR_OK) return bail(st);
-    if ((st = dev_upload(c, (noor_float4**)&S.nrm, P->normals, P->num_vertices)) != NOOR_OK) return bail(st);
-    if ((st = dev_upload(c, (noor_float2**)&S.uv, P->uvs, P->num_vertices)) != NOOR_OK) return bail(st);
     {
         std::vector<noor_float4> xf((size_t)9 * (P->num_instances ? P->num_instances : 1));
         for (uint32_t i = 0; i < P->num_instances; ++i)

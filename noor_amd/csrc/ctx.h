@@ -154,6 +154,10 @@ hipError_t launch_debug_skydome(const Context& c, uint32_t frame);
 hipError_t launch_sky_bake(const Context& c, float4* out, int w, int h);
 hipError_t launch_dist_build(const Context& c, const float4* tex, int tw, int th, float* func, float* cdf, int W,
                              int H);
+// Fills S.tri and S.shade (device arrays of 3 and 4 float4 per triangle) from
+// the payload's arrays on the device; `inst` may be null.
+hipError_t launch_tri_records(const Context& c, const uint4* attr, const float4* vert, const float4* nrm,
+                              const float2* uv, const uint32_t* ids, const uint32_t* inst);
 // kernels_adjoint.hip
 hipError_t launch_set_params(const Context& c, const float* albedo, const float* rough, uint32_t n, const float* env_rgb);
 // `radiance_lo`: the forward's direct_lo for the same sample, or null

@@ -88,15 +88,31 @@ __device__ __forceinline__ float dot3(f3 a, f3 b) { return a.x * b.x + a.y * b.y
 __device__ __forceinline__ f3 cross3(f3 a, f3 b) {
     return f3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
-__device__ __forceinline__ float len3(f3 a) { return sqrtf(dot3(a, a)); }
+// sqrt(x) and 1 / sqrt(x) as the IEEE square root and division round them, in
+// about half their instructions: for x in [2^-100, inf) one fused step on
+// x rsq(x) gives the correctly rounded root, and one on rcp(root) the correctly
+// rounded reciprocal (all such values compared on MI355X); the others take the
+// library's path.
+__device__ __forceinline__ bool root_range(float x) { return __float_as_uint(x) - 0x0D800000u < 0x72000000u; }
+__device__ __forceinline__ float root_step(float x) {
+    const float y = __builtin_amdgcn_rsqf(x), s = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+}
+__device__ __forceinline__ float fsqrt(float x) { return root_range(x) ? root_step(x) : sqrtf(x); }
+__device__ __forceinline__ float inv_sqrt(float x) {
+    if (!root_range(x)) return 1.0f / sqrtf(x);
+    const float s = root_step(x), y = __builtin_amdgcn_rcpf(s);
+    return __builtin_fmaf(__builtin_fmaf(-s, y, 1.0f), y, y);
+}
+__device__ __forceinline__ float len3(f3 a) { return fsqrt(dot3(a, a)); }
 __device__ __forceinline__ f3 nrm3(f3 a) {
-    const float inv = 1.0f / sqrtf(dot3(a, a));
+    const float inv = inv_sqrt(dot3(a, a));
     return scl3(a, inv);
 }
 __device__ __forceinline__ f3 nrm3s(f3 a) {
     const float l = dot3(a, a);
     if (l == 0.0f) return a;
-    const float inv = 1.0f / sqrtf(l);
+    const float inv = inv_sqrt(l);
     return scl3(a, inv);
 }
 __device__ __forceinline__ float absdot3(f3 a, f3 b) { return fabsf(dot3(a, b)); }
@@ -152,10 +168,12 @@ struct DevScene {
     const uint4* __restrict__ wald2;
     const float4* __restrict__ tri;      // v0, v1, v2 per triangle; their w: caller's triangle id, instance (of a
                                          // flat mesh's triangle), material type
-    const uint4* __restrict__ attr;
-    const float4* __restrict__ vert;
-    const float4* __restrict__ nrm;
-    const float2* __restrict__ uv;
+    // shading record, four float4 per triangle in leaf order: the vertex normals
+    // n0, n1, n2 (xyz of the first three), uv0 and uv1.x in their w, then uv1.y,
+    // uv2.x, uv2.y and the material index.  With the vertices above, one and a
+    // half memory lines hold what a hit needs; gathered through the vertex
+    // indices it was up to eleven, the second half of them after the first.
+    const float4* __restrict__ shade;
     const float4* __restrict__ xf;       // 9 rows per instance: w2o, o2w, normal
     const DevMat* __restrict__ mats;
     const float4* __restrict__ tex_texels;  // mip chains of the material textures
@@ -467,6 +485,25 @@ __device__ __forceinline__ uint32_t tri_word(const DevScene& S, uint32_t i, uint
 __device__ __forceinline__ uint32_t tri_id(const DevScene& S, uint32_t i) { return tri_word(S, i, 0); }
 __device__ __forceinline__ uint32_t tri_inst(const DevScene& S, uint32_t i) { return tri_word(S, i, 1); }
 __device__ __forceinline__ uint32_t tri_type(const DevScene& S, uint32_t i) { return tri_word(S, i, 2); }
+// A triangle's shading record (DevScene::shade).
+struct TriShade {
+    f3 n0, n1, n2;
+    f2 uv0, uv1, uv2;
+    uint32_t mat;
+};
+__device__ __forceinline__ TriShade load_shade(const DevScene& S, uint32_t i) {
+    const float4* p = S.shade + 4 * (size_t)i;
+    const float4 a = ldg(p), b = ldg(p + 1), c = ldg(p + 2), d = ldg(p + 3);
+    TriShade t;
+    t.n0 = f3{a.x, a.y, a.z};
+    t.n1 = f3{b.x, b.y, b.z};
+    t.n2 = f3{c.x, c.y, c.z};
+    t.uv0 = f2{a.w, b.w};
+    t.uv1 = f2{c.w, d.x};
+    t.uv2 = f2{d.y, d.z};
+    t.mat = __float_as_uint(d.w);
+    return t;
+}
 
 struct Counters {
     uint32_t nodes, tris, tri2, inst;
@@ -1126,12 +1163,12 @@ __device__ __forceinline__ float4 tex_point(const DevScene& S, uint32_t ti, floa
 
 // MaterialManager::getAlpha at the hit's interpolated uv (noor/cuda/materialimp.cuh:159-163)
 __device__ __forceinline__ bool alpha_pass(const DevScene& S, uint32_t tri, float u, float v) {
-    const uint4 ai = ldg(S.attr + tri);
-    const float2 q0 = ldg(S.uv + ai.x), q1 = ldg(S.uv + ai.y), q2 = ldg(S.uv + ai.z);
+    const TriShade T = load_shade(S, tri);
+    const f2 q0 = T.uv0, q1 = T.uv1, q2 = T.uv2;
     const float w = 1.0f - u - v;
     const float tu = w * q0.x + u * q1.x + v * q2.x;
     const float tv = w * (1.0f - q0.y) + u * (1.0f - q1.y) + v * (1.0f - q2.y);
-    const DevMat* m = S.mats + ai.w;
+    const DevMat* m = S.mats + T.mat;
     const float a = tex_point(S, m->tex[TX_ALPHA], m->uvs[TX_ALPHA][0] * tu, m->uvs[TX_ALPHA][1] * tv).x;
     return !(a <= 0.0001f);
 }
@@ -1321,9 +1358,13 @@ __device__ __forceinline__ void make_isect(const DevScene& S, const Ray& ray, co
         return;
     }
     I.tri = h.prim;
-    I.type = tri_type(S, h.prim);
-    const uint4 ai = ldg(S.attr + I.tri);
-    I.mat = ai.w;
+    const float4* V = S.tri + 3 * (size_t)h.prim;
+    const f3 p0 = fromf4(ldg(V)), p1 = fromf4(ldg(V + 1));
+    const float4 v2 = ldg(V + 2);
+    const f3 p2 = fromf4(v2);
+    I.type = __float_as_uint(v2.w);
+    const TriShade R = load_shade(S, I.tri);
+    I.mat = R.mat;
     if (I.type & M_EMITTER_ANY) {
         // an emitter keeps the barycentrics as its uv (computeTangentSpace
         // returns before interpolating, noor/cuda/intersection.cuh:326-327)
@@ -1333,10 +1374,8 @@ __device__ __forceinline__ void make_isect(const DevScene& S, const Ray& ray, co
         }
         return;
     }
-    const float2 q0 = ldg(S.uv + ai.x), q1 = ldg(S.uv + ai.y), q2 = ldg(S.uv + ai.z);
-    const f2 uv0 = f2{q0.x, 1.0f - q0.y}, uv1 = f2{q1.x, 1.0f - q1.y}, uv2 = f2{q2.x, 1.0f - q2.y};
-    const f3 p0 = fromf4(ldg(S.vert + ai.x)), p1 = fromf4(ldg(S.vert + ai.y)), p2 = fromf4(ldg(S.vert + ai.z));
-    const f3 n0 = fromf4(ldg(S.nrm + ai.x)), n1 = fromf4(ldg(S.nrm + ai.y)), n2 = fromf4(ldg(S.nrm + ai.z));
+    const f2 uv0 = f2{R.uv0.x, 1.0f - R.uv0.y}, uv1 = f2{R.uv1.x, 1.0f - R.uv1.y}, uv2 = f2{R.uv2.x, 1.0f - R.uv2.y};
+    const f3 n0 = R.n0, n1 = R.n1, n2 = R.n2;
     const float4* X = S.xf + 9 * (size_t)I.ins;
     Xf T = xf_load(X + 6);
     T.t = f3{0.0f, 0.0f, 0.0f};

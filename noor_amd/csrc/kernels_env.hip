@@ -113,4 +113,37 @@ hipError_t launch_dist_build(const Context& c, const float4* tex, int tw, int th
     return hipGetLastError();
 }
 
+// The per-triangle records the traversal and the shading read (DevScene::tri,
+// DevScene::shade), gathered once when a scene is created.
+__global__ void k_tri_records(const uint4* __restrict__ attr, const float4* __restrict__ vert,
+                              const float4* __restrict__ nrm, const float2* __restrict__ uv,
+                              const uint4* __restrict__ wald2, const uint32_t* __restrict__ ids,
+                              const uint32_t* __restrict__ inst, uint32_t n, float4* __restrict__ tri,
+                              float4* __restrict__ shade) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const uint4 a = attr[i];
+    const float4 p0 = vert[a.x], p1 = vert[a.y], p2 = vert[a.z];
+    const float4 n0 = nrm[a.x], n1 = nrm[a.y], n2 = nrm[a.z];
+    const float2 t0 = uv[a.x], t1 = uv[a.y], t2 = uv[a.z];
+    float4* T = tri + 3 * (size_t)i;
+    T[0] = make_float4(p0.x, p0.y, p0.z, __uint_as_float(ids[i]));
+    T[1] = make_float4(p1.x, p1.y, p1.z, __uint_as_float(inst ? inst[i] : 0u));
+    T[2] = make_float4(p2.x, p2.y, p2.z, __uint_as_float(wald2[i].w));
+    float4* R = shade + 4 * (size_t)i;
+    R[0] = make_float4(n0.x, n0.y, n0.z, t0.x);
+    R[1] = make_float4(n1.x, n1.y, n1.z, t0.y);
+    R[2] = make_float4(n2.x, n2.y, n2.z, t1.x);
+    R[3] = make_float4(t1.y, t2.x, t2.y, __uint_as_float(a.w));
+}
+
+hipError_t launch_tri_records(const Context& c, const uint4* attr, const float4* vert, const float4* nrm,
+                              const float2* uv, const uint32_t* ids, const uint32_t* inst) {
+    const uint32_t n = c.S.num_tris;
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_tri_records, dim3((n + 255) / 256), dim3(256), 0, c.stream, attr, vert, nrm, uv, c.S.wald2,
+                       ids, inst, n, const_cast<float4*>(c.S.tri), const_cast<float4*>(c.S.shade));
+    return hipGetLastError();
+}
+
 }  // namespace noor
