@@ -573,6 +573,7 @@ noor_status noor_create(const noor_payload_view* P, const noor_hosek* hosek, con
     if ((st = dev_upload(c, (noor::DevScene**)&c->d_scene, (const noor::DevScene*)nullptr, 1)) != NOOR_OK) return bail(st);
     if ((st = dev_upload(c, (noor::DevStats**)&c->d_stats, (const noor::DevStats*)nullptr, 1)) != NOOR_OK) return bail(st);
     if ((st = dev_upload(c, (float4**)&c->d_lookat, (const float4*)nullptr, 1)) != NOOR_OK) return bail(st);
+    if ((st = dev_upload(c, (noor::TileWork**)&c->d_tile_work, (const noor::TileWork*)nullptr, 1)) != NOOR_OK) return bail(st);
     if ((st = apply_options(c, options)) != NOOR_OK) return bail(st);
     if ((st = apply_spec(c, spec)) != NOOR_OK) return bail(st);
     if ((st = apply_camera(c, camera)) != NOOR_OK) return bail(st);

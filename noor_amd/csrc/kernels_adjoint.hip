@@ -33,6 +33,8 @@ struct AdjArgs {
     uint32_t stream;         // RNG stream (frame number) of the forward sample
 };
 
+// waves per SIMD: the box's 512x512 sample takes 0.80 ms, 0.92 at three, 0.98 at two
+constexpr int kAdjWaves = 4;
 constexpr uint32_t kLdsMats = 64;  // materials whose terms are summed in LDS first
 
 __device__ __forceinline__ void add_env(const DevScene& S, float* g, f3 dir, f3 wgt) {
@@ -70,7 +72,8 @@ __device__ __forceinline__ bool is_env_light(const DevScene& S, int idx) {
            S.skydome_type == NOOR_SKY_HDR;
 }
 
-__global__ __launch_bounds__(64) void k_adjoint(const DevScene* __restrict__ Sp, AdjArgs A) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kAdjWaves))) void k_adjoint(const DevScene* __restrict__ Sp, AdjArgs A,
+                                                                                                 TileWork* work, int lg) {
     const DevScene& S = *Sp;
     extern __shared__ uint32_t smem[];
     __shared__ float lmat[kLdsMats * 4];
@@ -78,15 +81,16 @@ __global__ __launch_bounds__(64) void k_adjoint(const DevScene* __restrict__ Sp,
     __syncthreads();
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t W = S.cam.w, H = S.cam.h;
-    const uint32_t tiles_x = (W + 7) / 8, tiles = tiles_x * ((H + 7) / 8);
+    const int lw = (lg + 1) / 2, lh = lg / 2;
+    const uint32_t tiles_x = (W + (1u << lw) - 1) >> lw, tiles = tiles_x * ((H + (1u << lh) - 1) >> lh);
     const TravStack st = make_stack(S, smem);
     Counters cnt{0, 0, 0, 0};
     bool overflow = false;
     float* genv = (S.sky_enabled && S.skydome_type == NOOR_SKY_HDR) ? A.g_env : nullptr;
-    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const uint32_t x = (tile % tiles_x) * 8 + (lane & 7);
-        const uint32_t y = (tile / tiles_x) * 8 + (lane >> 3);
-        if (x >= W || y >= H) continue;
+    for (uint32_t tile = blockIdx.x; tile < tiles; tile = next_tile(work)) {
+        const uint32_t x = ((tile % tiles_x) << lw) + (lane & ((1u << lw) - 1u));
+        const uint32_t y = ((tile / tiles_x) << lh) + (lane >> lw);
+        if (lane >> lg || x >= W || y >= H) continue;
         const uint32_t gid = y * W + x;
         const float4 g4 = A.grad[gid];
         const f3 dl = f3{g4.x, g4.y, g4.z};
@@ -153,6 +157,7 @@ __global__ __launch_bounds__(64) void k_adjoint(const DevScene* __restrict__ Sp,
             ps.bounce++;
         }
     }
+    tiles_done(work);
     __syncthreads();
     const uint32_t n = min(A.num_mats, kLdsMats);
     for (uint32_t i = threadIdx.x; i < n * 4; i += blockDim.x) {
@@ -207,12 +212,12 @@ hipError_t launch_adjoint(const Context& c, uint32_t stream, const float* radian
     A.g_env = g_env;
     A.num_mats = num_mats;
     A.stream = stream;
-    const uint32_t tiles = ((c.S.cam.w + 7) / 8) * ((c.S.cam.h + 7) / 8);
-    const uint32_t blocks = std::min<uint32_t>(tiles, c.S.gstack_lanes / 64);
+    const TileGrid g = tile_grid(c.S.cam.w, c.S.cam.h, c.S.gstack_lanes / (64 * 8) * kAdjWaves);
+    const uint32_t blocks = g.blocks;
     const size_t lds = (size_t)64 * c.S.stack_lds * sizeof(uint32_t);
     KernelTimer& T = const_cast<KernelTimer&>(c.timer);
     T.begin(c.stream, "adjoint");
-    hipLaunchKernelGGL(k_adjoint, dim3(blocks), dim3(64), lds, c.stream, c.d_scene, A);
+    hipLaunchKernelGGL(k_adjoint, dim3(blocks), dim3(64), lds, c.stream, c.d_scene, A, c.d_tile_work, g.lg);
     T.end(c.stream);
     return hipGetLastError();
 }

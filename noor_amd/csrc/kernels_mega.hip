@@ -1,7 +1,8 @@
 // Megakernel renderer (the drop-in for path_tracer_kernel,
 // noor/cuda/path_tracer.cu:77-100) and the hit-query test hook.
 //
-// Launch shape: 1-D blocks of 64 lanes; each wave renders an 8x8 pixel tile
+// Launch shape: 1-D blocks of 64 lanes; each wave renders an 8x8 pixel tile (a
+// smaller one of a small image)
 // so that primary rays of a wave are coherent.  A launch renders `spp`
 // progressive frames and keeps the pixel's film value in registers between
 // them; the per-frame running mean is applied in frame order, so the film is
@@ -44,27 +45,34 @@ __device__ __forceinline__ void flush_stats(DevStats* st, unsigned long long ext
 
 // DIRECT: write each pixel's last sample to `direct` instead of updating the
 // film (a separate instantiation keeps the film path's register budget).
-// Two waves per SIMD are required: at one the latency of the traversal's
-// node loads is exposed and the kernel runs about 1.7x slower.
-// TEX: image textures, alpha tests, bump and ray differentials.
+// Held to four waves per SIMD: the spills (outside the traversal's loop) cost less
+// than the waits that the third and fourth wave hide.  512x512x4 samples of the
+// box take 2.6 ms, 3.2 at two or three waves, 4.1 at five; the 1080p terrain frame
+// 3.0 ms, 4.6 at two, 3.1 at three and five.  Lanes that take the next sample or
+// pixel as soon as theirs ends, instead of with their wave, gain nothing (2.8 and
+// 3.0 ms): the mixed rays cost what the fuller waves save.
+// TEX: image textures, alpha tests, bump and ray differentials; two waves (256
+// VGPRs with spills already).
+constexpr int kMegaWaves = 4;
 template <bool STATS, bool DIRECT, bool TEX = false>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_megakernel(const DevScene* __restrict__ Sp, float4* __restrict__ film, uint32_t frame0,
-                                                   uint32_t spp, DevStats* __restrict__ stats,
-                                                   float4* __restrict__ lookat_out, float4* __restrict__ direct,
-                                                   float4* __restrict__ direct_lo) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(TEX ? 2 : kMegaWaves))) void k_megakernel(
+    const DevScene* __restrict__ Sp, float4* __restrict__ film, uint32_t frame0, uint32_t spp,
+    DevStats* __restrict__ stats, float4* __restrict__ lookat_out, float4* __restrict__ direct,
+    float4* __restrict__ direct_lo, TileWork* __restrict__ work, int lg) {
     const DevScene& S = *Sp;
     extern __shared__ uint32_t smem[];
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t W = S.cam.w, H = S.cam.h;
-    const uint32_t tiles_x = (W + 7) / 8, tiles = tiles_x * ((H + 7) / 8);
+    const int lw = (lg + 1) / 2, lh = lg / 2;
+    const uint32_t tiles_x = (W + (1u << lw) - 1) >> lw, tiles = tiles_x * ((H + (1u << lh) - 1) >> lh);
     const TravStack st = make_stack(S, smem);
     Counters cnt{0, 0, 0, 0}, cns{0, 0, 0, 0};
     unsigned long long ext = 0, shd = 0, nhit = 0;
     bool overflow = false;
-    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const uint32_t x = (tile % tiles_x) * 8 + (lane & 7);
-        const uint32_t y = (tile / tiles_x) * 8 + (lane >> 3);
-        if (x >= W || y >= H) continue;
+    for (uint32_t tile = blockIdx.x; tile < tiles; tile = next_tile(work)) {
+        const uint32_t x = ((tile % tiles_x) << lw) + (lane & ((1u << lw) - 1u));
+        const uint32_t y = ((tile / tiles_x) << lh) + (lane >> lw);
+        if (lane >> lg || x >= W || y >= H) continue;
         const uint32_t gid = y * W + x;
         float4 acc = DIRECT ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : film[gid];
         // the autofocus point of the centre pixel's last sample: its first hit,
@@ -118,34 +126,34 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
         else film[gid] = acc;
         if (center && lookat_out) *lookat_out = lookat;
     }
+    tiles_done(work);
     flush_stats(stats, ext, shd, nhit, cnt, cns, overflow);
 }
 
 hipError_t launch_megakernel(const Context& c, uint32_t frame0, uint32_t spp, float4* direct, float4* direct_lo) {
     hipError_t se = sync_scene(c);
     if (se != hipSuccess) return se;
-    const uint32_t tiles = ((c.S.cam.w + 7) / 8) * ((c.S.cam.h + 7) / 8);
-    // one wave per 8x8 tile, grid-stride over tiles within the lanes the global stack covers
-    const uint32_t blocks = std::min<uint32_t>(tiles, c.S.gstack_lanes / 64);
+    const TileGrid g = tile_grid(c.S.cam.w, c.S.cam.h, c.S.gstack_lanes / (64 * 8) * (c.S.textured ? 2 : kMegaWaves));
+    const uint32_t blocks = g.blocks;  // within the lanes the global stack covers
     const size_t lds = (size_t)64 * c.S.stack_lds * sizeof(uint32_t);
     KernelTimer& T = const_cast<KernelTimer&>(c.timer);
     T.begin(c.stream, "megakernel");
     if (direct && c.S.textured) return hipErrorNotSupported;
     if (direct)
         hipLaunchKernelGGL((k_megakernel<false, true>), dim3(blocks), dim3(64), lds, c.stream, c.d_scene, c.film, frame0,
-                           spp, c.d_stats, c.d_lookat, direct, direct_lo);
+                           spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.lg);
     else if (c.S.textured && c.opt.stats)
         hipLaunchKernelGGL((k_megakernel<true, false, true>), dim3(blocks), dim3(64), lds, c.stream, c.d_scene, c.film,
-                           frame0, spp, c.d_stats, c.d_lookat, direct, direct_lo);
+                           frame0, spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.lg);
     else if (c.S.textured)
         hipLaunchKernelGGL((k_megakernel<false, false, true>), dim3(blocks), dim3(64), lds, c.stream, c.d_scene, c.film,
-                           frame0, spp, c.d_stats, c.d_lookat, direct, direct_lo);
+                           frame0, spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.lg);
     else if (c.opt.stats)
         hipLaunchKernelGGL((k_megakernel<true, false>), dim3(blocks), dim3(64), lds, c.stream, c.d_scene, c.film, frame0,
-                           spp, c.d_stats, c.d_lookat, direct, direct_lo);
+                           spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.lg);
     else
         hipLaunchKernelGGL((k_megakernel<false, false>), dim3(blocks), dim3(64), lds, c.stream, c.d_scene, c.film, frame0,
-                           spp, c.d_stats, c.d_lookat, direct, direct_lo);
+                           spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.lg);
     T.end(c.stream);
     return hipGetLastError();
 }
