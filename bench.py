@@ -19,7 +19,7 @@ bytes count the events of the reference's binary-BVH traversal of the same
 rays, from the oracle's counters over the CPU sample: 32 B per node visit,
 32 B per triangle test plus 16 B when the second Wald record is read, 48 B per
 instance entry (per extension ray, scaled to the step's extension rays).
-`achieved_build_layout` counts the renderer's own fetches instead (56 B per
+`achieved_build_layout` counts the renderer's own fetches instead (64 B per
 compressed wide-node visit, 48 B per watertight triangle test, 48 B per
 instance entry, 72 B of queue and record traffic per ray).  `traffic` and
 `limiter` are the HBM bytes per dispatch (FETCH_SIZE + WRITE_SIZE, scaled by a
@@ -55,7 +55,7 @@ sys.path.insert(0, ROOT)
 
 METRIC = "Mrays/s + spp/s @1080p (wavefront vs megakernel); bwd/fwd time ratio"
 HBM_PEAK_GBS = 8000.0
-WIDE_NODE_BYTES = 56  # per wide-node visit: origin + steps (16 B), 8-bit child planes (24 B), references (16 B)
+WIDE_NODE_BYTES = 64  # per wide-node visit: origin + steps (24 B), 8-bit child planes (24 B), references (16 B)
 PMC_PROFILE = os.path.join(ROOT, "profiles", "pmc_traffic_terrain_1080p.md")
 
 
@@ -117,15 +117,15 @@ def shade_roofline(st, paths, kt, prof):
     beta) and written (L, beta, RNG: 40); per continuing ray the next ray and
     its queue entry (36); per shadow task the NEE candidate, shadow ray and
     queue entry (68); per ended path its free-queue entry (4); per hit the
-    shading fetch (attributes 16, three vertices, normals and uvs 120,
-    object-to-world and normal rows 96: 232) and the material record (128);
+    shading fetch (the triangle's two records 112, object-to-world and normal
+    rows 96: 208) and the material record (128);
     per miss the environment lookup (64)."""
     if "wave_shade" not in kt:
         return None
     # (the totals below are over every path; the last factor keeps k_shade's share)
     ext, shd, hits = st["extension_rays"], st["shadow_rays"], st["extension_hits"]
     cont = ext - paths  # every extension ray after a path's first
-    total = (ext * (116 + 40) - paths * 32 + cont * 36 + shd * 68 + paths * 4 + hits * (232 + 128) +
+    total = (ext * (116 + 40) - paths * 32 + cont * 36 + shd * 68 + paths * 4 + hits * (208 + 128) +
              (ext - hits) * 64)
     # k_shade shades the hits of the rays k_extend traced (the drain the rest)
     total *= (ext - st["drain_extension_rays"]) / max(1, ext)
@@ -601,7 +601,7 @@ def main():
                 "rays_per_launch": int((ext_k if dom == "wave_extend" else shd_k) / launches),
                 "limiter": ({"valu_rate": kprof["valu_rate"], "lanes_active": kprof["lanes_active"],
                              "wave_wait_fraction": kprof["wave_wait_fraction"],
-                             "what": f"latency of the traversal's dependent fetches with "
+                             "what": f"VALU instructions of the traversal's steps with "
                                      f"{100 * kprof['lanes_active']:.0f}% of the lanes active "
                                      "(hardware counters, see traffic source)"}
                             if kprof else None),

@@ -302,14 +302,19 @@ noor_status build_environment(Context* c) {
     const int W = std::min(std::max(nearest_pow2(tw), 32), 1024);
     const int H = std::min(std::max(nearest_pow2(th), 32), 1024);
     const size_t n = (size_t)H * (W + 2) + 1;
-    if (c->dfunc) hipFree(c->dfunc);
-    if (c->dcdf) hipFree(c->dcdf);
-    c->dfunc = c->dcdf = nullptr;
-    void* p = nullptr;
-    HIP_TRY(c, hipMalloc(&p, sizeof(float) * n));
-    c->dfunc = (float*)p;
-    HIP_TRY(c, hipMalloc(&p, sizeof(float) * n));
-    c->dcdf = (float*)p;
+    // the arrays are kept between calls of one size (new parameters every
+    // optimiser step): freeing and allocating them took 0.15 ms of each
+    if (!c->dfunc || !c->dcdf || c->dist_n != n) {
+        if (c->dfunc) hipFree(c->dfunc);
+        if (c->dcdf) hipFree(c->dcdf);
+        c->dfunc = c->dcdf = nullptr;
+        c->dist_n = n;
+        void* p = nullptr;
+        HIP_TRY(c, hipMalloc(&p, sizeof(float) * n));
+        c->dfunc = (float*)p;
+        HIP_TRY(c, hipMalloc(&p, sizeof(float) * n));
+        c->dcdf = (float*)p;
+    }
     HIP_TRY(c, hipMemsetAsync(c->dfunc, 0, sizeof(float) * n, c->stream));
     HIP_TRY(c, hipMemsetAsync(c->dcdf, 0, sizeof(float) * n, c->stream));
     HIP_TRY(c, noor::launch_dist_build(*c, tex, tw, th, c->dfunc, c->dcdf, W, H));
@@ -406,26 +411,34 @@ noor_status noor_create(const noor_payload_view* P, const noor_hosek* hosek, con
     if ((st = dev_upload(c, (noor_uint4**)&S.wald2, P->wald_cnu_cnv_deg_mat, nt)) != NOOR_OK) return bail(st);
     {
         // per-triangle records, gathered on the device from the payload's vertex arrays, which are not kept
-        noor_uint4* attr = nullptr;
-        noor_float4 *vert = nullptr, *nrm = nullptr;
-        noor_float2* uv = nullptr;
-        uint32_t *ids = nullptr, *inst = nullptr;
+        // (one temporary allocation: each hipFree waits for the device)
         std::vector<uint32_t> count_up;
         if (!P->prim_ids) {
             count_up.resize(nt);
             for (uint32_t i = 0; i < nt; ++i) count_up[i] = i;
         }
-        const size_t kept = c->allocs.size();
-        if ((st = dev_upload(c, &attr, P->attribute_indices, nt)) != NOOR_OK) return bail(st);
-        if ((st = dev_upload(c, &vert, P->vertices, P->num_vertices)) != NOOR_OK) return bail(st);
-        if ((st = dev_upload(c, &nrm, P->normals, P->num_vertices)) != NOOR_OK) return bail(st);
-        if ((st = dev_upload(c, &uv, P->uvs, P->num_vertices)) != NOOR_OK) return bail(st);
-        if ((st = dev_upload(c, &ids, P->prim_ids ? P->prim_ids : count_up.data(), nt)) != NOOR_OK) return bail(st);
-        if (!flat_inst.empty() && (st = dev_upload(c, &inst, flat_inst.data(), nt)) != NOOR_OK) return bail(st);
-        const std::vector<void*> temporary(c->allocs.begin() + kept, c->allocs.end());
-        c->allocs.resize(kept);
+        const struct {
+            const void* src;
+            size_t bytes;
+        } parts[] = {{P->attribute_indices, sizeof(noor_uint4) * (size_t)nt},
+                     {P->vertices, sizeof(noor_float4) * (size_t)P->num_vertices},
+                     {P->normals, sizeof(noor_float4) * (size_t)P->num_vertices},
+                     {P->uvs, sizeof(noor_float2) * (size_t)P->num_vertices},
+                     {P->prim_ids ? P->prim_ids : count_up.data(), sizeof(uint32_t) * (size_t)nt},
+                     {flat_inst.data(), sizeof(uint32_t) * flat_inst.size()}};
+        size_t at[6], total = 256;
+        for (int k = 0; k < 6; ++k) {
+            at[k] = total;
+            total += (parts[k].bytes + 255) & ~(size_t)255;
+        }
+        void* temporary = nullptr;
+        hipError_t e = hipMalloc(&temporary, total);
+        for (int k = 0; k < 6 && e == hipSuccess; ++k)
+            if (parts[k].bytes)
+                e = hipMemcpyAsync((char*)temporary + at[k], parts[k].src, parts[k].bytes, hipMemcpyHostToDevice,
+                                   c->stream);
         void *tri = nullptr, *shade = nullptr;
-        hipError_t e = hipMalloc(&tri, sizeof(float4) * 3 * (size_t)std::max(nt, 1u));
+        if (e == hipSuccess) e = hipMalloc(&tri, sizeof(float4) * 3 * (size_t)std::max(nt, 1u));
         if (e == hipSuccess) {
             c->allocs.push_back(tri);
             e = hipMalloc(&shade, sizeof(float4) * 4 * (size_t)std::max(nt, 1u));
@@ -434,11 +447,15 @@ noor_status noor_create(const noor_payload_view* P, const noor_hosek* hosek, con
             c->allocs.push_back(shade);
             S.tri = (const float4*)tri;
             S.shade = (const float4*)shade;
-            e = noor::launch_tri_records(*c, (const uint4*)attr, (const float4*)vert, (const float4*)nrm,
-                                         (const float2*)uv, ids, inst);
+            const char* t = (const char*)temporary;
+            e = noor::launch_tri_records(*c, (const uint4*)(t + at[0]), (const float4*)(t + at[1]),
+                                         (const float4*)(t + at[2]), (const float2*)(t + at[3]),
+                                         (const uint32_t*)(t + at[4]),
+                                         flat_inst.empty() ? nullptr : (const uint32_t*)(t + at[5]));
         }
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        for (void* p : temporary) hipFree(p);
+        const hipError_t es = hipStreamSynchronize(c->stream);  // also before the temporary goes
+        if (e == hipSuccess) e = es;
+        hipFree(temporary);
         if (e != hipSuccess)
             return bail(fail(c, e == hipErrorOutOfMemory ? NOOR_ERR_OUT_OF_MEMORY : NOOR_ERR_HIP,
                              std::string("triangle records: ") + hipGetErrorString(e)));
@@ -596,6 +613,7 @@ noor_status noor_destroy(noor_ctx* ctx) {
     if (c->sample_lo) hipFree(c->sample_lo);
     if (c->dfunc) hipFree(c->dfunc);
     if (c->dcdf) hipFree(c->dcdf);
+    if (c->trace_buf) hipFree(c->trace_buf);
     if (c->stream) hipStreamDestroy(c->stream);
     delete ctx;
     return NOOR_OK;
@@ -992,23 +1010,41 @@ noor_status noor_synchronize(noor_ctx* ctx) {
     return NOOR_OK;
 }
 
+constexpr size_t kTraceKeep = (size_t)64 << 20;  // bytes of rays and hits a context keeps between noor_trace calls
+
 noor_status noor_trace(noor_ctx* ctx, const noor_ray* rays, uint32_t n, int any_hit, noor_hit* hits) {
     if (!ctx || !rays || !hits) return NOOR_ERR_INVALID_ARG;
     if (n == 0) return NOOR_OK;
     Context* c = &ctx->c;
-    void *dr = nullptr, *dh = nullptr;
-    HIP_TRY(c, hipMalloc(&dr, sizeof(noor_ray) * n));
-    hipError_t e = hipMalloc(&dh, sizeof(noor_hit) * n);
-    if (e != hipSuccess) {
-        hipFree(dr);
-        return fail(c, NOOR_ERR_OUT_OF_MEMORY, "hit buffer");
+    // Rays, then hits, in a buffer the context keeps up to kTraceKeep; larger
+    // batches allocate for the call.
+    const size_t off = (sizeof(noor_ray) * (size_t)n + 255) & ~(size_t)255, need = off + sizeof(noor_hit) * (size_t)n;
+    char* buf = (char*)c->trace_buf;
+    if (need > c->trace_bytes) {
+        void* p = nullptr;
+        if (need <= kTraceKeep && c->trace_buf) {
+            HIP_TRY(c, hipFree(c->trace_buf));
+            c->trace_buf = nullptr;
+            c->trace_bytes = 0;
+        }
+        if (hipMalloc(&p, need) != hipSuccess) {
+            (void)hipGetLastError();
+            return fail(c, NOOR_ERR_OUT_OF_MEMORY, "ray and hit buffers");
+        }
+        buf = (char*)p;
+        if (need <= kTraceKeep) {
+            c->trace_buf = p;
+            c->trace_bytes = need;
+        }
     }
-    e = hipMemcpyAsync(dr, rays, sizeof(noor_ray) * n, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = noor::launch_trace(*c, (const noor_ray*)dr, n, any_hit, (noor_hit*)dh);
-    if (e == hipSuccess) e = hipMemcpyAsync(hits, dh, sizeof(noor_hit) * n, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    hipFree(dr);
-    hipFree(dh);
+    noor_ray* dr = (noor_ray*)buf;
+    noor_hit* dh = (noor_hit*)(buf + off);
+    hipError_t e = hipMemcpyAsync(dr, rays, sizeof(noor_ray) * (size_t)n, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = noor::launch_trace(*c, dr, n, any_hit, dh);
+    if (e == hipSuccess) e = hipMemcpyAsync(hits, dh, sizeof(noor_hit) * (size_t)n, hipMemcpyDeviceToHost, c->stream);
+    const hipError_t es = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = es;
+    if (buf != (char*)c->trace_buf) hipFree(buf);
     if (e != hipSuccess) return fail(c, NOOR_ERR_HIP, std::string("trace: ") + hipGetErrorString(e));
     return NOOR_OK;
 }

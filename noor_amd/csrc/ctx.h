@@ -112,6 +112,9 @@ struct Context {
     float4* sky_bake = nullptr;
     float* dfunc = nullptr;
     float* dcdf = nullptr;
+    size_t dist_n = 0;            // floats in each
+    void* trace_buf = nullptr;    // noor_trace's rays and hits
+    size_t trace_bytes = 0;
     noor_hosek* d_hosek = nullptr;
     DevStats* d_stats = nullptr;
     float4* d_lookat = nullptr;
