@@ -156,7 +156,9 @@ inline hipError_t sync_scene(const Context& cc) {
 // waves per SIMD is cut into smaller ones: its waves run fewer lanes each, but
 // in fewer different branches and on more of the GPU (64 x 64 pixels of the box,
 // one sample: 0.34 ms with 64-pixel tiles at two waves per SIMD, 0.25 with
-// 1- or 2-pixel tiles, 0.33 with 4-pixel ones).
+// 1- or 2-pixel tiles, 0.33 with 4-pixel ones), and no more of them than waves
+// fit at once (a second, mostly empty round cost the adjoint 0.73 against 0.53 ms
+// at 300 x 200 pixels).
 // The launch has as many blocks as the GPU holds at once; a wave that is done
 // with its tile takes the next one of the launch (with the tiles dealt out in
 // advance the 1080p terrain frame takes 3.6 instead of 3.0 ms).
@@ -166,7 +168,7 @@ struct TileGrid {
 };
 inline TileGrid tile_grid(uint32_t w, uint32_t h, uint32_t waves) {
     int lg = 6;
-    while (lg > 1 && ((uint64_t)w * h >> lg) < waves) --lg;
+    while (lg > 1 && ((uint64_t)w * h >> (lg - 1)) <= waves) --lg;
     const uint32_t tw = 1u << ((lg + 1) / 2), th = 1u << (lg / 2);
     const uint32_t tiles = ((w + tw - 1) / tw) * ((h + th - 1) / th);
     return TileGrid{tiles < waves ? tiles : waves, lg};
