@@ -893,7 +893,9 @@ __device__ __forceinline__ bool trav_steps(const DevScene& S, Trav& t, const Tra
             }
         } else if (kind == REF_INST) {
             next = ldg(S.inst_root + t.ins);
-            t.leaves = (next & REF_TLAS) ? REF_LEAVES_FLAT : REF_TLAS;
+            // (REF_EMPTY, a mesh without triangles, has the TLAS bit but is no flat mesh: what is popped next
+            // may be one, in the world's space)
+            t.leaves = next != REF_EMPTY && (next & REF_TLAS) ? REF_LEAVES_FLAT : REF_TLAS;
         } else if (cur != REF_EMPTY) {  // (an empty scene's root)
             // light nodes are top-level references: lray is the world ray here
             const uint32_t li = cur & REF_INDEX_MASK;

@@ -73,3 +73,45 @@ def test_flat_meshes_match_oracle(layout):
     np.testing.assert_array_equal(mega, orc.render(1, 2)[0])
     r.render_wavefront(2, frame=1)
     np.testing.assert_array_equal(mega, r.film())
+
+
+def _empty_instance(placement):
+    """A sphere placed by the identity, beside an instance of a mesh without triangles whose box is finite and in the
+    way of the sphere's rays."""
+    sb = SceneBuilder()
+    m = sb.add_material(material(abi.MAT_DIFFUSE, diffuse=(0.6, 0.5, 0.4)))
+    sv, sf = scenes.icosphere(3)
+    a = sb.add_mesh(Mesh(sv * 0.4, sf, normals=sv, material=m))
+    b = sb.add_mesh(Mesh(np.array([[-1.0, -1.0, -1.0], [1.0, 1.0, 1.0], [1.0, -1.0, 1.0]]), np.array([[0, 1, 2]]),
+                         material=m))
+    sb.add_instance(a, EYE)
+    sb.add_instance(b, placement)
+    sb.set_env(scenes.env_map(64, 32, 5))
+    payload = sb.build()
+    nodes = payload.arrays()
+    leaf, only = 0x80000000, 0x80000001  # triangle leaves of the node format: the flag, and the count in the low bits
+    one = np.flatnonzero(nodes["bvh_b"][:, 3] == only)
+    one = [i for i in one if nodes["attr"][nodes["bvh_a"][i, 3], 0] >= len(sv)]  # the second mesh's
+    assert len(one) == 1
+    nodes["bvh_b"][one[0], 3] = leaf
+    cam = make_camera((0.0, 1.2, 2.6), (0.0, 0.0, 0.0), (0, 1, 0), np.radians(50.0), 61, 47)
+    return scenes.Workload("empty", payload, cam, make_spec(payload, bounces=4), make_options(), None, 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("placement", [TURN, SHIFT, EYE], ids=["turned", "shifted", "identity"])
+def test_empty_instance_beside_a_flat_mesh(placement):
+    wl = _empty_instance(placement)
+    assert lib().noor_wide_bvh_check(C.byref(wl.payload.view), None, None) == abi.OK
+    g = np.random.default_rng(42)
+    o = g.normal(size=(5000, 3))
+    o *= 3.0 / np.linalg.norm(o, axis=1, keepdims=True)
+    rays = rays_from_numpy(o.astype(np.float32), (g.uniform(-0.4, 0.4, (5000, 3)) - o).astype(np.float32))
+    r, orc = Renderer.from_workload(wl), OracleScene.from_workload(wl)
+    hits = hits_to_numpy(r.trace(rays))
+    assert (hits[:, 6] > 0).sum() > 1000
+    np.testing.assert_array_equal(hits, hits_to_numpy(orc.trace(rays)[0]))
+    np.testing.assert_array_equal(hits_to_numpy(r.trace(rays, any_hit=True))[:, 6],
+                                  hits_to_numpy(orc.trace(rays, any_hit=True)[0])[:, 6])
+    r.render_wavefront(2)
+    np.testing.assert_array_equal(r.film(), orc.render(1, 2)[0])
