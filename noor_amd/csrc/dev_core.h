@@ -432,7 +432,8 @@ __device__ __forceinline__ void box4_hit_exact(const Ray& r, const WideNode& n, 
         const float tz1 = (q_plane(oz, fz, c, sz) - r.o.z) * r.inv.z;
         const float t0 = fmaxf(fmaxf(tx0, ty0), tz0);
         const float t1 = fminf(fminf(tx1, ty1), tz1) * BOX_SLACK;
-        tn[c] = t0 <= t1 && t0 <= tmaxs && t1 >= 0.0f ? t0 : K_INF;
+        // (a box reached at an infinite distance, by a direction so short that its reciprocal overflows, is entered)
+        tn[c] = t0 <= t1 && t0 <= tmaxs && t1 >= 0.0f ? fminf(t0, __FLT_MAX__) : K_INF;
     }
 }
 

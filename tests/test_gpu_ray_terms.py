@@ -40,3 +40,16 @@ def test_scaled_directions_bit_exact(pair, axis, exponent, any_hit):
         np.testing.assert_array_equal(g[:, 6], h[:, 6])
     else:
         np.testing.assert_array_equal(g, h)
+
+
+@pytest.mark.parametrize("exponent", [-129, -131, -135])
+def test_overflowing_reciprocals_enter_boxes(pair, exponent):
+    """Directions whose reciprocals overflow reach every box in front of them at an infinite distance: the boxes are
+    entered as the reference's comparison does, and the hits, themselves at infinity, are those of the oracle."""
+    r, orc = pair
+    o, d = _rays(33)
+    rays = rays_from_numpy(o, d * np.float32(2.0 ** exponent))
+    g, h = hits_to_numpy(r.trace(rays)), hits_to_numpy(orc.trace(rays)[0])
+    assert (h[:, 6] > 0).sum() > 1000
+    np.testing.assert_array_equal(g, h)
+    assert (hits_to_numpy(r.trace(rays, any_hit=True))[h[:, 6] > 0, 6] > 0).all()
