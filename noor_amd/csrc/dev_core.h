@@ -304,8 +304,8 @@ __device__ __forceinline__ void ray_update_box(Ray& r) {
 // Intersection", JCGT 2(1), 2013 (axis permutation and shear).  Needs inv.
 // The permutation is a rotation, z the dominant axis; the paper's exchange of x
 // and y for a negative d[z] is left out: it only negates U, V, W and the
-// determinant together, which leaves the test, t, u and v as they are but for
-// the sign of a zero (tri_watertight restores it).
+// determinant together, which leaves the test, t, u and v as they are
+// (tri_watertight sees to the signs of zeros).
 __device__ __forceinline__ float perm_x(f3 v, bool z0, bool z1) { return z0 ? v.y : (z1 ? v.z : v.x); }
 __device__ __forceinline__ float perm_y(f3 v, bool z0, bool z1) { return z0 ? v.z : (z1 ? v.x : v.y); }
 __device__ __forceinline__ float perm_z(f3 v, bool z0, bool z1) { return z0 ? v.x : (z1 ? v.y : v.z); }
@@ -560,9 +560,14 @@ __device__ __forceinline__ bool tri_watertight(const DevScene& S, const Ray& r, 
     float V = Ax * Cy - Ay * Cx;
     float W = Bx * Ay - By * Ax;
     if (U == 0.0f || V == 0.0f || W == 0.0f) {
-        U = (float)((double)Cx * (double)By - (double)Cy * (double)Bx);
-        V = (float)((double)Ax * (double)Cy - (double)Ay * (double)Cx);
-        W = (float)((double)Bx * (double)Ay - (double)By * (double)Ax);
+        // (the negated difference of the exchanged products, for a negative d[z]: a zero keeps the sign it has there)
+        auto edge = [&](float px, float qy, float py, float qx) {
+            const double a = (double)px * (double)qy, b = (double)py * (double)qx;
+            return (float)(r.Sz < 0.0f ? -(b - a) : a - b);
+        };
+        U = edge(Cx, By, Cy, Bx);
+        V = edge(Ax, Cy, Ay, Cx);
+        W = edge(Bx, Ay, By, Ax);
     }
     if ((U < 0.0f || V < 0.0f || W < 0.0f) && (U > 0.0f || V > 0.0f || W > 0.0f)) return false;
     const float det = U + V + W;
@@ -575,13 +580,8 @@ __device__ __forceinline__ bool tri_watertight(const DevScene& S, const Ray& r, 
     to = t;
     uo = V * inv;
     vo = W * inv;
-    if (r.Sz < 0.0f) {
-        // x and y not exchanged: a zero edge function, or a sum that cancelled
-        // to zero, has the sign +0 either way while 1 / det has the other one
-        if (V == 0.0f) uo = -uo;
-        if (W == 0.0f) vo = -vo;
-        if (Tt == 0.0f && (U * Az != 0.0f || V * Bz != 0.0f)) to = -to;
-    }
+    // x and y not exchanged: all terms are the negatives, but terms that cancel add up to +0 either way
+    if (Tt == 0.0f && r.Sz < 0.0f) to = (-(U * Az) - V * Bz - W * Cz) * -inv;
     return true;
 }
 

@@ -5,6 +5,7 @@ import pytest
 
 from noor_amd import abi, scenes
 from noor_amd.renderer import Renderer, hits_to_numpy, rays_from_numpy
+from noor_amd.scene import Mesh, SceneBuilder, make_camera, make_options, make_spec, material
 from oracle.binding import OracleScene
 
 pytestmark = pytest.mark.gpu
@@ -53,3 +54,29 @@ def test_overflowing_reciprocals_enter_boxes(pair, exponent):
     assert (h[:, 6] > 0).sum() > 1000
     np.testing.assert_array_equal(g, h)
     assert (hits_to_numpy(r.trace(rays, any_hit=True))[h[:, 6] > 0, 6] > 0).all()
+
+
+@pytest.mark.parametrize("exact", [True, False])
+def test_signs_of_zeros(exact):
+    """Rays from and through a mesh's vertices and edges along coordinate planes: edge functions, distances and
+    barycentrics of zero have the oracle's sign."""
+    v, t = scenes.icosphere(2)
+    sb = SceneBuilder()
+    sb.add_mesh(Mesh(v * 0.5, t, normals=v, material=sb.add_material(material(abi.MAT_DIFFUSE))))
+    sb.set_env(scenes.env_map(64, 32, 5))
+    payload = sb.build()
+    wl = scenes.Workload("ball", payload, make_camera((0.0, 0.0, 3.0), (0.0, 0.0, 0.0), (0, 1, 0), 1.0, 16, 16),
+                         make_spec(payload, bounces=2), make_options(), None, 1)
+    g = np.random.default_rng(44)
+    p = payload.arrays()["vertices"][:, :3]
+    tgt = p[g.integers(0, len(p), 6000)]
+    d = g.integers(-3, 4, (6000, 3)).astype(np.float32)
+    d[(d == 0).any(1)] += np.float32(0.5)
+    # origins on the vertices, or (an exact multiple of the direction away) rays through them
+    o = tgt if exact else (tgt - d * np.float32(0.5)).astype(np.float32)
+    rays = rays_from_numpy(o, d)
+    hits = hits_to_numpy(Renderer.from_workload(wl).trace(rays))
+    want = hits_to_numpy(OracleScene.from_workload(wl).trace(rays)[0])
+    zero = want[want[:, 6] > 0, :3] & 0x7FFFFFFF == 0
+    assert zero.sum() > (3000 if exact else 100)
+    np.testing.assert_array_equal(hits, want)
