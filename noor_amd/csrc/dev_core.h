@@ -764,9 +764,12 @@ __device__ __forceinline__ void trav_begin(const DevScene& S, const Ray& r, Trav
     t.d = r.d;
     t.lray = r;
     t.leaves = 0u;
-    // zero, tiny, huge, infinite or NaN components: flat meshes through their instance
-    const float z = r.o.x * 0.0f + r.o.y * 0.0f + r.o.z * 0.0f;
-    t.cur = (r.pn & 16u) && z == 0.0f ? S.wroot : S.wroot_strict;
+    // flat meshes through their instance where the identity changes the ray: direction components that are zero (or
+    // tiny, huge, infinite; NaN ones hit no triangle either way), origin components that are -0, infinite or NaN
+    constexpr int kOdd = 0x227;
+    const bool odd = __builtin_isfpclass(r.o.x, kOdd) || __builtin_isfpclass(r.o.y, kOdd) ||
+                     __builtin_isfpclass(r.o.z, kOdd);
+    t.cur = (r.pn & 16u) && !odd ? S.wroot : S.wroot_strict;
     t.ins = 0;
     t.sp = 0;
     t.kind = 0;

@@ -115,3 +115,23 @@ def test_empty_instance_beside_a_flat_mesh(placement):
                                   hits_to_numpy(orc.trace(rays, any_hit=True)[0])[:, 6])
     r.render_wavefront(2)
     np.testing.assert_array_equal(r.film(), orc.render(1, 2)[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["both_flat", "flat_and_turned"])
+def test_origins_with_negative_zeros(layout):
+    """Origins on the sphere's vertices, their zeros written as -0, which the identity's product turns into +0: hits
+    at distance zero keep the sign the oracle gives them."""
+    wl = _workload(layout)
+    sv, _ = scenes.icosphere(3)
+    sv = (sv * 0.4).astype(np.float32)
+    sv = sv[(sv == 0.0).any(1)]
+    g = np.random.default_rng(43)
+    o = sv[g.integers(0, len(sv), 4000)]
+    o = np.where(o == 0.0, np.float32(-0.0), o)
+    rays = rays_from_numpy(o, g.normal(size=(4000, 3)).astype(np.float32))
+    for tri in (abi.TRI_WATERTIGHT, abi.TRI_WALD):
+        wl.options.tri_test = tri
+        hits = hits_to_numpy(Renderer.from_workload(wl).trace(rays))
+        assert (hits[:, 6] > 0).sum() > 1000
+        np.testing.assert_array_equal(hits, hits_to_numpy(OracleScene.from_workload(wl).trace(rays)[0]))
