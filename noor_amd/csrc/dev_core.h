@@ -835,9 +835,13 @@ __device__ __forceinline__ bool trav_steps(const DevScene& S, Trav& t, const Tra
             if (STATS) c.nodes++;
             const WideNode n = load_wnode(S, cur & REF_NODE_MASK);
             float d[4];
-            box4_hit(t.lray, n, d);
-            if (__ballot(!(t.lray.pn & 8u)) != 0ull) {
-                if (!(t.lray.pn & 8u)) box4_hit_exact(t.lray, n, d);
+            // A wave of axis-parallel rays runs the exact form only.  With the fast one for all lanes first, 2M such
+            // queries took 0.57 instead of 0.48 ms (box) and 0.83 instead of 0.70 (terrain).
+            if (__builtin_expect(__ballot(!(t.lray.pn & 8u)) == 0ull, 1)) {
+                box4_hit(t.lray, n, d);
+            } else {
+                if (t.lray.pn & 8u) box4_hit(t.lray, n, d);
+                else box4_hit_exact(t.lray, n, d);
             }
             float d0 = d[0], d1 = __uint_as_float(n.b.y) > 0.0f ? d[1] : K_INF;
             float d2 = __uint_as_float(n.b.x) > 0.0f ? d[2] : K_INF, d3 = n.a.w > 0.0f ? d[3] : K_INF;

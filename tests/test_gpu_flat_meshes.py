@@ -135,3 +135,29 @@ def test_origins_with_negative_zeros(layout):
         hits = hits_to_numpy(Renderer.from_workload(wl).trace(rays))
         assert (hits[:, 6] > 0).sum() > 1000
         np.testing.assert_array_equal(hits, hits_to_numpy(OracleScene.from_workload(wl).trace(rays)[0]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["both_flat", "flat_and_turned", "none_flat"])
+@pytest.mark.parametrize("per_wave", [1, 32, 63, 64])
+def test_axis_rays_in_a_wave(layout, per_wave):
+    """Rays with zero or very small direction components (the exact box test, the strict top level) as the only ones of
+    their wave, as some of it and as all but one."""
+    wl = _workload(layout)
+    g = np.random.default_rng(45)
+    n = 64 * 150
+    o = g.normal(size=(n, 3))
+    o *= 1.4 / np.linalg.norm(o, axis=1, keepdims=True)  # below the light: a light just behind an origin counts as hit
+    d = g.uniform(-0.4, 0.4, (n, 3)) - o
+    lanes = np.argsort(g.random((n // 64, 64)), axis=1).ravel() < per_wave  # that many random lanes of each wave
+    small = g.choice([0.0, 2.0 ** -100, -2.0 ** -100, -2.0 ** -130], (n, 3))
+    axis = g.integers(0, 3, n)
+    put = lanes[:, None] & (np.arange(3)[None] == axis[:, None])
+    o, d = np.where(put, g.uniform(-0.3, 0.3, (n, 3)), o), np.where(put, small, d)
+    rays = rays_from_numpy(o.astype(np.float32), d.astype(np.float32))
+    r, orc = Renderer.from_workload(wl), OracleScene.from_workload(wl)
+    hits = hits_to_numpy(r.trace(rays))
+    assert (hits[lanes, 6] > 0).sum() > lanes.sum() // 8
+    np.testing.assert_array_equal(hits, hits_to_numpy(orc.trace(rays)[0]))
+    np.testing.assert_array_equal(hits_to_numpy(r.trace(rays, any_hit=True))[:, 6],
+                                  hits_to_numpy(orc.trace(rays, any_hit=True)[0])[:, 6])
