@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "dev_core.h"
+#include "tile_feed.h"
 
 namespace noor {
 
@@ -26,14 +27,6 @@ struct DevStats {
     unsigned long long shd[4];
     unsigned long long overflow;
     unsigned long long ext_hits;  // closest-hit queries that hit (counted with STATS)
-};
-
-// Tiles handed out beyond each block's first (TileFeed), and blocks that have
-// ended: the last block of a launch clears both, so a launch needs no memset
-// before it.  Each on a 256-byte line of its own.
-struct TileWork {
-    uint32_t next, pad0[63];
-    uint32_t done, pad1[63];
 };
 
 struct WaveBuffers;  // wavefront queues (kernels_wave.hip)
@@ -159,9 +152,6 @@ inline hipError_t sync_scene(const Context& cc) {
 // 1- or 2-pixel tiles, 0.33 with 4-pixel ones), and no more of them than waves
 // fit at once (a second, mostly empty round cost the adjoint 0.73 against 0.53 ms
 // at 300 x 200 pixels).
-// The launch has as many blocks as the GPU holds at once; a wave that is done
-// with its tile takes the next one of the launch (with the tiles dealt out in
-// advance the 1080p terrain frame takes 3.6 instead of 3.0 ms).
 struct TileGrid {
     uint32_t blocks;
     int lg;
@@ -171,22 +161,8 @@ inline TileGrid tile_grid(uint32_t w, uint32_t h, uint32_t waves) {
     while (lg > 1 && ((uint64_t)w * h >> (lg - 1)) <= waves) --lg;
     const uint32_t tw = 1u << ((lg + 1) / 2), th = 1u << (lg / 2);
     const uint32_t tiles = ((w + tw - 1) / tw) * ((h + th - 1) / th);
-    return TileGrid{tiles < waves ? tiles : waves, lg};
+    return TileGrid{tile_blocks(tiles, waves), lg};
 }
-#ifdef __HIPCC__
-// The tiles of a one-wave block: its own first, then from the launch's counter.
-__device__ __forceinline__ uint32_t next_tile(TileWork* work) {
-    uint32_t n = 0;
-    if ((threadIdx.x & 63u) == 0) n = atomicAdd(&work->next, 1u);
-    return gridDim.x + (uint32_t)__builtin_amdgcn_readfirstlane((int)n);
-}
-// Every block calls it once, after its last next_tile().
-__device__ __forceinline__ void tiles_done(TileWork* work) {
-    if ((threadIdx.x & 63u) != 0 || atomicAdd(&work->done, 1u) != gridDim.x - 1u) return;
-    atomicExch(&work->next, 0u);
-    atomicExch(&work->done, 0u);
-}
-#endif
 // kernels_mega.hip
 // `direct`: write each pixel's last sample there instead of updating the film
 // `direct_lo` (DIRECT only, may be null): the rounding error of each sample's

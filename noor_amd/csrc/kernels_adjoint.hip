@@ -87,7 +87,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kAdjWaves)))
     Counters cnt{0, 0, 0, 0};
     bool overflow = false;
     float* genv = (S.sky_enabled && S.skydome_type == NOOR_SKY_HDR) ? A.g_env : nullptr;
-    for (uint32_t tile = blockIdx.x; tile < tiles; tile = next_tile(work)) {
+    for (uint32_t tile = first_tile(tiles); tile < tiles; tile = next_tile(work, tiles)) {
         const uint32_t x = ((tile % tiles_x) << lw) + (lane & ((1u << lw) - 1u));
         const uint32_t y = ((tile / tiles_x) << lh) + (lane >> lw);
         if (lane >> lg || x >= W || y >= H) continue;
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kAdjWaves)))
             ps.bounce++;
         }
     }
-    tiles_done(work);
+    tiles_done(work, tiles);
     __syncthreads();
     const uint32_t n = min(A.num_mats, kLdsMats);
     for (uint32_t i = threadIdx.x; i < n * 4; i += blockDim.x) {

@@ -69,7 +69,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(TEX ? 2 : kM
     Counters cnt{0, 0, 0, 0}, cns{0, 0, 0, 0};
     unsigned long long ext = 0, shd = 0, nhit = 0;
     bool overflow = false;
-    for (uint32_t tile = blockIdx.x; tile < tiles; tile = next_tile(work)) {
+    for (uint32_t tile = first_tile(tiles); tile < tiles; tile = next_tile(work, tiles)) {
         const uint32_t x = ((tile % tiles_x) << lw) + (lane & ((1u << lw) - 1u));
         const uint32_t y = ((tile / tiles_x) << lh) + (lane >> lw);
         if (lane >> lg || x >= W || y >= H) continue;
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(TEX ? 2 : kM
         else film[gid] = acc;
         if (center && lookat_out) *lookat_out = lookat;
     }
-    tiles_done(work);
+    tiles_done(work, tiles);
     flush_stats(stats, ext, shd, nhit, cnt, cns, overflow);
 }
 

@@ -25,3 +25,14 @@ def test_tiles_cover_the_image(renderer, w, h, spp):
     for _ in range(3):  # the tile counters are back at zero after each launch
         renderer.render(spp, frame=1)
         np.testing.assert_array_equal(renderer.film(), want)
+
+
+def test_groups_that_run_out_take_from_the_others(renderer):
+    """An image whose rows cost very different times (sky above, the box's inside below), with many tiles per block and
+    a remainder in every direction, several times in a row."""
+    renderer.update_camera(make_camera((0.0, 0.9, 3.0), (0.0, 1.2, -1.0), (0, 1, 0), np.radians(80.0), 2051, 1027))
+    renderer.render_wavefront(1, frame=1)
+    want = renderer.film()
+    for _ in range(3):
+        renderer.render(1, frame=1)
+        np.testing.assert_array_equal(renderer.film(), want)
