@@ -803,13 +803,11 @@ __device__ __forceinline__ uint32_t leaf_next(uint32_t cur) {
     return ((cur >> REF_LEAF_COUNT_SHIFT) & 7u) ? cur + 1u - (1u << REF_LEAF_COUNT_SHIFT) : REF_EMPTY;
 }
 
-//
-// KIND: a closest-hit query, an any-hit one (ends at the first triangle or light
-// it finds, t.hit()), or the lane's choice in `any`.
-enum : int { TRAV_CLOSEST, TRAV_ANY, TRAV_MIXED };
-template <bool STATS, bool ALPHA, int KIND>
+// ANY: an any-hit query, which ends at the first triangle or light it finds
+// (t.hit()).
+template <bool STATS, bool ALPHA, bool ANY>
 __device__ __forceinline__ bool trav_steps(const DevScene& S, Trav& t, const TravStack& st, Counters& c,
-                                           bool& overflow, int max_steps, bool any = KIND == TRAV_ANY) {
+                                           bool& overflow, int max_steps) {
     bool done = false;
     for (int step = 0; step < max_steps && !done; ++step) {
         const uint32_t cur = t.cur;
@@ -874,7 +872,7 @@ __device__ __forceinline__ bool trav_steps(const DevScene& S, Trav& t, const Tra
             next = leaf_next(cur);
             float tt, u, v;
             if (tri_test<STATS, ALPHA>(S, t.lray, ti, tt, u, v, c)) {
-                if (KIND != TRAV_CLOSEST && any) {
+                if (ANY) {
                     t.kind = 1;
                     t.sp = 0;
                     next = REF_EMPTY;
@@ -909,7 +907,7 @@ __device__ __forceinline__ bool trav_steps(const DevScene& S, Trav& t, const Tra
             const uint32_t li = cur & REF_INDEX_MASK;
             Ray tr = t.lray;
             const bool lh = light_node_intersect(S, li, tr);
-            if (KIND != TRAV_CLOSEST && any) {
+            if (ANY) {
                 if (lh) {
                     t.kind = 1;
                     t.sp = 0;
@@ -941,7 +939,7 @@ __device__ __forceinline__ bool bvh_closest(const DevScene& S, Ray& ray, Hit& h,
                                             bool& overflow) {
     Trav t;
     trav_begin(S, ray, t);
-    while (!trav_steps<STATS, ALPHA, TRAV_CLOSEST>(S, t, st, c, overflow, 1 << 30)) {
+    while (!trav_steps<STATS, ALPHA, false>(S, t, st, c, overflow, 1 << 30)) {
     }
     ray.tmax = t.lray.tmax;
     h = trav_hit(S, t);
@@ -953,7 +951,7 @@ __device__ __forceinline__ bool bvh_any(const DevScene& S, const Ray& ray, const
                                         bool& overflow) {
     Trav t;
     trav_begin(S, ray, t);
-    while (!trav_steps<STATS, ALPHA, TRAV_ANY>(S, t, st, c, overflow, 1 << 30)) {
+    while (!trav_steps<STATS, ALPHA, true>(S, t, st, c, overflow, 1 << 30)) {
     }
     return t.hit();
 }

@@ -449,7 +449,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
             have = true;
         }
         if (__ballot(have) == 0ull) break;
-        if (have && trav_steps<STATS, ALPHA, TRAV_CLOSEST>(S, t, st, cnt, overflow, B.steps)) {
+        if (have && trav_steps<STATS, ALPHA, false>(S, t, st, cnt, overflow, B.steps)) {
             const Hit h = trav_hit(S, t);
             const uint32_t p = q[qi >> 3];
             B.hit[2 * (size_t)p] = make_uint4(__float_as_uint(h.t), __float_as_uint(h.u), __float_as_uint(h.v), h.prim);
@@ -714,7 +714,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
             ++shd;
         }
         if (__ballot(have) == 0ull) break;
-        if (have && trav_steps<STATS, ALPHA, TRAV_ANY>(S, t, st, cnt, overflow, B.steps)) {
+        if (have && trav_steps<STATS, ALPHA, true>(S, t, st, cnt, overflow, B.steps)) {
             const bool nb = MIS && B.nee_b[p].w != 0.0f;
             if (!second && nb) {
                 occ_a = t.hit();
