@@ -411,6 +411,14 @@ noor_status noor_render_sample(noor_ctx* ctx, uint32_t stream, float* radiance);
 noor_status noor_adjoint(noor_ctx* ctx, uint32_t stream, const float* radiance, const float* grad_image,
                          float* grad_albedo, float* grad_roughness, uint32_t num_materials, float* grad_env);
 
+/* Compares the kernels' short forms of correctly rounded operations with the
+ * compiler's IEEE division and square root on the current GPU, over all 2^32
+ * floats: op 0 the reciprocal, 1 the square root, 2 the reciprocal of the square
+ * root; over 2^32 pairs of magnitudes from 2^-60 to 2^60: op 3 the quotient from
+ * a reciprocal; op 4 the hardware's reciprocal estimate alone, which does
+ * differ.  Counts the results that differ in any bit (NaNs count as equal). */
+noor_status noor_rounding_check(int op, uint64_t* differences);
+
 /* Host-side check of the four-wide BVH the traversal kernels use (no GPU
  * needed): builds it from a payload and verifies that every triangle of every
  * instanced BLAS is reachable exactly once per BLAS, that every child box

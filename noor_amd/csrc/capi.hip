@@ -920,6 +920,21 @@ noor_status noor_adjoint(noor_ctx* ctx, uint32_t stream, const float* radiance, 
     return NOOR_OK;
 }
 
+noor_status noor_rounding_check(int op, uint64_t* differences) {
+    if (!differences || op < 0 || op > 4) return NOOR_ERR_INVALID_ARG;
+    if (noor_device_count() == 0) return NOOR_ERR_NO_DEVICE;
+    void* d = nullptr;
+    unsigned long long n = 0;
+    if (hipMalloc(&d, sizeof(n)) != hipSuccess) return NOOR_ERR_OUT_OF_MEMORY;
+    hipError_t e = hipMemcpy(d, &n, sizeof(n), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = noor::launch_rounding(op, (unsigned long long*)d);
+    if (e == hipSuccess) e = hipMemcpy(&n, d, sizeof(n), hipMemcpyDeviceToHost);
+    (void)hipFree(d);
+    if (e != hipSuccess) return NOOR_ERR_HIP;
+    *differences = n;
+    return NOOR_OK;
+}
+
 noor_status noor_wide_bvh_check(const noor_payload_view* P, uint32_t* num_nodes, uint32_t* stack_need_out) {
     if (!P) return NOOR_ERR_INVALID_ARG;
     Context tmp;

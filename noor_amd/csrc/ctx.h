@@ -186,6 +186,7 @@ hipError_t launch_dist_build(const Context& c, const float4* tex, int tw, int th
 // the payload's arrays on the device; `inst` may be null.
 hipError_t launch_tri_records(const Context& c, const uint4* attr, const float4* vert, const float4* nrm,
                               const float2* uv, const uint32_t* ids, const uint32_t* inst);
+hipError_t launch_rounding(int op, unsigned long long* differences);  // adds to a device counter
 // kernels_adjoint.hip
 hipError_t launch_set_params(const Context& c, const float* albedo, const float* rough, uint32_t n, const float* env_rgb);
 // `radiance_lo`: the forward's direct_lo for the same sample, or null

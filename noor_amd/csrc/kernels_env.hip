@@ -146,4 +146,39 @@ hipError_t launch_tri_records(const Context& c, const uint4* attr, const float4*
     return hipGetLastError();
 }
 
+// noor_rounding_check: element i of an operation against its IEEE form.
+template <int OP>
+__device__ __forceinline__ bool rounds_alike(uint32_t i) {
+    const float x = __uint_as_float(i);
+    float got, want;
+    if (OP == 0) got = frcp(x), want = 1.0f / x;
+    if (OP == 1) got = fsqrt(x), want = sqrtf(x);
+    if (OP == 2) got = inv_sqrt(x), want = 1.0f / sqrtf(x);
+    if (OP == 3) {
+        // all 2^23 fractions of the divisor, with 512 dividends and pairs of exponents (67 ... 187 is 2^-60 ... 2^60)
+        const uint32_t h = (i * 0x9E3779B1u) ^ (i >> 15) * 0x85EBCA77u;
+        const float a = __uint_as_float((h & 0x807FFFFFu) | (67u + (h >> 24) % 120u) << 23);
+        const float b = __uint_as_float((i & 0x007FFFFFu) | (67u + (i >> 23) % 120u) << 23);
+        got = div_by_rcp(a, b, 1.0f / b), want = a / b;
+    }
+    if (OP == 4) got = __builtin_amdgcn_rcpf(x), want = 1.0f / x;
+    return __float_as_uint(got) == __float_as_uint(want) || (got != got && want != want);
+}
+template <int OP>
+__global__ void k_rounding(unsigned long long* differences) {
+    const uint32_t step = gridDim.x * blockDim.x;  // divides 2^32
+    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, n = 0;
+    for (uint64_t k = 0; k < (1ull << 32) / step; ++k, i += step) n += rounds_alike<OP>(i) ? 0u : 1u;
+    if (n) atomicAdd(differences, (unsigned long long)n);
+}
+hipError_t launch_rounding(int op, unsigned long long* differences) {
+    const dim3 grid(4096), block(256);
+    if (op == 0) hipLaunchKernelGGL(k_rounding<0>, grid, block, 0, 0, differences);
+    else if (op == 1) hipLaunchKernelGGL(k_rounding<1>, grid, block, 0, 0, differences);
+    else if (op == 2) hipLaunchKernelGGL(k_rounding<2>, grid, block, 0, 0, differences);
+    else if (op == 3) hipLaunchKernelGGL(k_rounding<3>, grid, block, 0, 0, differences);
+    else hipLaunchKernelGGL(k_rounding<4>, grid, block, 0, 0, differences);
+    return hipGetLastError();
+}
+
 }  // namespace noor
