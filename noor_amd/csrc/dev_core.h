@@ -91,7 +91,7 @@ __device__ __forceinline__ f3 cross3(f3 a, f3 b) {
 // sqrt(x) and 1 / sqrt(x) as the IEEE square root and division round them, in
 // about half their instructions: for x in [2^-100, inf) one fused step on
 // x rsq(x) gives the correctly rounded root, and one on rcp(root) the correctly
-// rounded reciprocal (all such values compared on MI355X); the others take the
+// rounded reciprocal (noor_rounding_check compares them all); the others take the
 // library's path.
 __device__ __forceinline__ bool root_range(float x) { return __float_as_uint(x) - 0x0D800000u < 0x72000000u; }
 __device__ __forceinline__ float root_step(float x) {
@@ -263,8 +263,8 @@ struct Ray {
 
 // 1 / x, correctly rounded as the IEEE division is, in half its instructions:
 // one fused Newton step on the hardware reciprocal gives the same bits for
-// every x whose hardware reciprocal is a normal number (all 2^32 values
-// compared with 1.0f / x on MI355X); the others take the division.
+// every x whose hardware reciprocal is a normal number (noor_rounding_check
+// compares all 2^32 values with 1.0f / x); the others take the division.
 __device__ __forceinline__ bool is_normal(float x) { return __builtin_isfpclass(x, 0x108); }
 __device__ __forceinline__ float rcp_step(float x, float y) { return __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y); }
 __device__ __forceinline__ float frcp(float x) {
