@@ -422,6 +422,11 @@ __device__ __forceinline__ void box4_hit_exact(const Ray& r, const WideNode& n, 
     const uint32_t ny = (r.pn & 2u) ? qhy : qly, fy = (r.pn & 2u) ? qly : qhy;
     const uint32_t nz = (r.pn & 4u) ? qhz : qlz, fz = (r.pn & 4u) ? qlz : qhz;
     const float tmaxs = r.tmax * BOX_SLACK;
+    // A box reached at an infinite distance, by a direction so short that its
+    // reciprocals overflow, is entered; a zero direction hits no triangle, and
+    // visiting all that lies ahead of it made four such rays of 2.3M take k_extend
+    // 4.6 instead of 1.1 ms.
+    const float most = r.d.x == 0.0f && r.d.y == 0.0f && r.d.z == 0.0f ? K_INF : __FLT_MAX__;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         const float tx0 = (q_plane(ox, nx, c, sx) - r.o.x) * r.inv.x;
@@ -432,8 +437,7 @@ __device__ __forceinline__ void box4_hit_exact(const Ray& r, const WideNode& n, 
         const float tz1 = (q_plane(oz, fz, c, sz) - r.o.z) * r.inv.z;
         const float t0 = fmaxf(fmaxf(tx0, ty0), tz0);
         const float t1 = fminf(fminf(tx1, ty1), tz1) * BOX_SLACK;
-        // (a box reached at an infinite distance, by a direction so short that its reciprocal overflows, is entered)
-        tn[c] = t0 <= t1 && t0 <= tmaxs && t1 >= 0.0f ? fminf(t0, __FLT_MAX__) : K_INF;
+        tn[c] = t0 <= t1 && t0 <= tmaxs && t1 >= 0.0f ? fminf(t0, most) : K_INF;
     }
 }
 

@@ -80,3 +80,21 @@ def test_signs_of_zeros(exact):
     zero = want[want[:, 6] > 0, :3] & 0x7FFFFFFF == 0
     assert zero.sum() > (3000 if exact else 100)
     np.testing.assert_array_equal(hits, want)
+
+
+def test_zero_directions_visit_little():
+    """A path can lose its direction.  Such a ray hits nothing, and the boxes ahead of it, all at an infinite distance,
+    are not searched: a few such rays would hold up a whole film."""
+    wl = scenes.cornell(subdiv=5, width=16, height=16)
+    wl.options.stats = 1
+    r, orc = Renderer.from_workload(wl), OracleScene.from_workload(wl)
+    o, _ = _rays(35)
+    d = np.where(np.random.default_rng(36).random(o.shape) < 0.5, np.float32(-0.0), np.float32(0.0))
+    rays = rays_from_numpy(o, d)
+    r.reset_stats()
+    hits = hits_to_numpy(r.trace(rays))
+    np.testing.assert_array_equal(hits, hits_to_numpy(orc.trace(rays)[0]))
+    assert (hits[:, 6] == 0).all()
+    assert r.stats()["node_visits"] < 64 * len(o)
+    np.testing.assert_array_equal(hits_to_numpy(r.trace(rays, any_hit=True))[:, 6],
+                                  hits_to_numpy(orc.trace(rays, any_hit=True)[0])[:, 6])
