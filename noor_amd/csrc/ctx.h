@@ -158,14 +158,15 @@ inline hipError_t sync_scene(const Context& cc) {
 // lines: 1 x 8000, 8,000 tiles, 0.29 against 0.27).
 struct TileGrid {
     uint32_t blocks;
-    int lg;
+    int feed;  // lg, and from bit 8 the blocks of each group (first_tile's `dealt`)
 };
 inline TileGrid tile_grid(uint32_t w, uint32_t h, uint32_t waves) {
     int lg = 6;
     while (lg > 1 && ((uint64_t)w * h >> (lg - 1)) <= waves) --lg;
     const uint32_t tw = 1u << ((lg + 1) / 2), th = 1u << (lg / 2);
     const uint32_t tiles = ((w + tw - 1) / tw) * ((h + th - 1) / th);
-    return TileGrid{tile_blocks(tiles, waves), lg};
+    const uint32_t blocks = tile_blocks(tiles, waves), dealt = blocks < tiles ? blocks / kTileGroups : 0u;
+    return TileGrid{blocks, lg | (int)(dealt << 8)};
 }
 // kernels_mega.hip
 // `direct`: write each pixel's last sample there instead of updating the film

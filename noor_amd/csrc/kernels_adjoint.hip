@@ -73,7 +73,7 @@ __device__ __forceinline__ bool is_env_light(const DevScene& S, int idx) {
 }
 
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kAdjWaves))) void k_adjoint(const DevScene* __restrict__ Sp, AdjArgs A,
-                                                                                                 TileWork* work, int lg) {
+                                                                                                 TileWork* work, int feed) {
     const DevScene& S = *Sp;
     extern __shared__ uint32_t smem[];
     __shared__ float lmat[kLdsMats * 4];
@@ -81,13 +81,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kAdjWaves)))
     __syncthreads();
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t W = S.cam.w, H = S.cam.h;
-    const int lw = (lg + 1) / 2, lh = lg / 2;
+    const int lg = feed & 255, lw = (lg + 1) / 2, lh = lg / 2;
+    const uint32_t dealt = (uint32_t)feed >> 8;
     const uint32_t tiles_x = (W + (1u << lw) - 1) >> lw, tiles = tiles_x * ((H + (1u << lh) - 1) >> lh);
     const TravStack st = make_stack(S, smem);
     Counters cnt{0, 0, 0, 0};
     bool overflow = false;
     float* genv = (S.sky_enabled && S.skydome_type == NOOR_SKY_HDR) ? A.g_env : nullptr;
-    for (uint32_t tile = first_tile(tiles); tile < tiles; tile = next_tile(work, tiles)) {
+    for (uint32_t tile = first_tile(dealt); tile < tiles; tile = next_tile(work, tiles, dealt)) {
         const uint32_t x = ((tile % tiles_x) << lw) + (lane & ((1u << lw) - 1u));
         const uint32_t y = ((tile / tiles_x) << lh) + (lane >> lw);
         if (lane >> lg || x >= W || y >= H) continue;
@@ -157,7 +158,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kAdjWaves)))
             ps.bounce++;
         }
     }
-    tiles_done(work, tiles);
+    tiles_done(work, dealt);
     __syncthreads();
     const uint32_t n = min(A.num_mats, kLdsMats);
     for (uint32_t i = threadIdx.x; i < n * 4; i += blockDim.x) {
@@ -217,7 +218,7 @@ hipError_t launch_adjoint(const Context& c, uint32_t stream, const float* radian
     const size_t lds = (size_t)64 * c.S.stack_lds * sizeof(uint32_t);
     KernelTimer& T = const_cast<KernelTimer&>(c.timer);
     T.begin(c.stream, "adjoint");
-    hipLaunchKernelGGL(k_adjoint, dim3(blocks), dim3(64), lds, c.stream, c.d_scene, A, c.d_tile_work, g.lg);
+    hipLaunchKernelGGL(k_adjoint, dim3(blocks), dim3(64), lds, c.stream, c.d_scene, A, c.d_tile_work, g.feed);
     T.end(c.stream);
     return hipGetLastError();
 }

@@ -58,18 +58,19 @@ template <bool STATS, bool DIRECT, bool TEX = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(TEX ? 2 : kMegaWaves))) void k_megakernel(
     const DevScene* __restrict__ Sp, float4* __restrict__ film, uint32_t frame0, uint32_t spp,
     DevStats* __restrict__ stats, float4* __restrict__ lookat_out, float4* __restrict__ direct,
-    float4* __restrict__ direct_lo, TileWork* __restrict__ work, int lg) {
+    float4* __restrict__ direct_lo, TileWork* __restrict__ work, int feed) {
     const DevScene& S = *Sp;
     extern __shared__ uint32_t smem[];
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t W = S.cam.w, H = S.cam.h;
-    const int lw = (lg + 1) / 2, lh = lg / 2;
+    const int lg = feed & 255, lw = (lg + 1) / 2, lh = lg / 2;
+    const uint32_t dealt = (uint32_t)feed >> 8;
     const uint32_t tiles_x = (W + (1u << lw) - 1) >> lw, tiles = tiles_x * ((H + (1u << lh) - 1) >> lh);
     const TravStack st = make_stack(S, smem);
     Counters cnt{0, 0, 0, 0}, cns{0, 0, 0, 0};
     unsigned long long ext = 0, shd = 0, nhit = 0;
     bool overflow = false;
-    for (uint32_t tile = first_tile(tiles); tile < tiles; tile = next_tile(work, tiles)) {
+    for (uint32_t tile = first_tile(dealt); tile < tiles; tile = next_tile(work, tiles, dealt)) {
         const uint32_t x = ((tile % tiles_x) << lw) + (lane & ((1u << lw) - 1u));
         const uint32_t y = ((tile / tiles_x) << lh) + (lane >> lw);
         if (lane >> lg || x >= W || y >= H) continue;
@@ -126,7 +127,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(TEX ? 2 : kM
         else film[gid] = acc;
         if (center && lookat_out) *lookat_out = lookat;
     }
-    tiles_done(work, tiles);
+    tiles_done(work, dealt);
     flush_stats(stats, ext, shd, nhit, cnt, cns, overflow);
 }
 
@@ -141,19 +142,19 @@ hipError_t launch_megakernel(const Context& c, uint32_t frame0, uint32_t spp, fl
     if (direct && c.S.textured) return hipErrorNotSupported;
     if (direct)
         hipLaunchKernelGGL((k_megakernel<false, true>), dim3(blocks), dim3(64), lds, c.stream, c.d_scene, c.film, frame0,
-                           spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.lg);
+                           spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.feed);
     else if (c.S.textured && c.opt.stats)
         hipLaunchKernelGGL((k_megakernel<true, false, true>), dim3(blocks), dim3(64), lds, c.stream, c.d_scene, c.film,
-                           frame0, spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.lg);
+                           frame0, spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.feed);
     else if (c.S.textured)
         hipLaunchKernelGGL((k_megakernel<false, false, true>), dim3(blocks), dim3(64), lds, c.stream, c.d_scene, c.film,
-                           frame0, spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.lg);
+                           frame0, spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.feed);
     else if (c.opt.stats)
         hipLaunchKernelGGL((k_megakernel<true, false>), dim3(blocks), dim3(64), lds, c.stream, c.d_scene, c.film, frame0,
-                           spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.lg);
+                           spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.feed);
     else
         hipLaunchKernelGGL((k_megakernel<false, false>), dim3(blocks), dim3(64), lds, c.stream, c.d_scene, c.film, frame0,
-                           spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.lg);
+                           spp, c.d_stats, c.d_lookat, direct, direct_lo, c.d_tile_work, g.feed);
     T.end(c.stream);
     return hipGetLastError();
 }

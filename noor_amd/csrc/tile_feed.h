@@ -19,12 +19,11 @@ namespace noor {
 // over kTileGroups groups with a counter each, block b taking from group
 // b % kTileGroups, one group per XCD: returning atomics on one address are
 // 11.7 ns apart, which with one counter made a frame whose rays all miss take
-// 0.40 ms at 1920x1080 and 1.51 at 3840x2160 (0.19 and 0.45 with 8 groups, 0.15
-// and 0.39 with 16, 0.10 and 0.29 with the tiles dealt out; 16 take 8.4 instead
-// of 8.2 ms for the terrain at 3840x2160, one 8.4).  A group owns one tile of
-// every kTileGroups, another one in each run of them, so that no group gets the
-// same columns of every row; a block whose group has run out takes from the
-// others.
+// 0.40 ms at 1920x1080 and 1.51 at 3840x2160 (0.15 and 0.40 with eight; 0.10 and
+// 0.29 with the tiles dealt out; sixteen made the terrain at 3840x2160 3%
+// slower).  A group owns one tile of every kTileGroups, another one in each run
+// of them, so that no group gets the same columns of every row; a block whose
+// group has run out takes from the others.
 constexpr uint32_t kTileGroups = 8;
 
 // Tile of entry i of group g, and the entries of a group.
@@ -52,39 +51,36 @@ struct TileWork {
 };
 
 #ifdef __HIPCC__
-// A one-wave block's first tile.
-__device__ __forceinline__ uint32_t first_tile(uint32_t tiles) {
-    if (gridDim.x >= tiles) return blockIdx.x;
+// `dealt`: the blocks of each group, or 0 when every tile is some block's first
+// and no counter is used (an argument of the launch: kept from the grid's size
+// it cost the megakernel registers and 3% with the Wald test).
+__device__ __forceinline__ uint32_t first_tile(uint32_t dealt) {
+    if (dealt == 0u) return blockIdx.x;
     return group_tile(blockIdx.x % kTileGroups, blockIdx.x / kTileGroups);
 }
-// Its next one; `tiles` when there is none.  Called by all lanes of the wave.
-__device__ __forceinline__ uint32_t next_tile(TileWork* work, uint32_t tiles) {
-    if (gridDim.x >= tiles) return tiles;  // every tile was some block's first
-    const uint32_t lane = threadIdx.x & 63u, dealt = gridDim.x / kTileGroups;  // (blocks of each group)
+// The block's next tile; `tiles` when there is none.  Called by all lanes of the
+// wave.
+__device__ __forceinline__ uint32_t next_tile(TileWork* work, uint32_t tiles, uint32_t dealt) {
+    if (dealt == 0u) return tiles;
     uint32_t g = blockIdx.x % kTileGroups;
-    // groups that may have tiles left: each turn takes a tile or one of them away
-    for (uint32_t left = (1u << kTileGroups) - 1u; left != 0u;) {
+    for (uint32_t k = 0; k < kTileGroups; ++k, g = (g + 1) % kTileGroups) {
+        const uint32_t size = group_size(g, tiles) - dealt;
+        // (another group's counter is read first: most have run out as well by then)
+        if (k != 0 && (uint32_t)__builtin_amdgcn_readfirstlane((int)__hip_atomic_load(
+                          &work->next[g].v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >= size)
+            continue;
         uint32_t n = 0;
-        if (lane == 0) n = atomicAdd(&work->next[g].v, 1u);
-        const uint32_t i = dealt + (uint32_t)__builtin_amdgcn_readfirstlane((int)n);
-        if (i < group_size(g, tiles)) return group_tile(g, i);
-        // this group has run out: look at all of them, take the next one that has not
-        left &= ~(1u << g);
-        bool some = false;
-        if (lane < kTileGroups)
-            some = dealt + __hip_atomic_load(&work->next[lane].v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
-                   group_size(lane, tiles);
-        left &= (uint32_t)__ballot(some);
-        const uint32_t after = left & ~((2u << g) - 1u);
-        g = (uint32_t)__builtin_ctz((after ? after : left) | (1u << kTileGroups));
+        if ((threadIdx.x & 63u) == 0) n = atomicAdd(&work->next[g].v, 1u);
+        n = (uint32_t)__builtin_amdgcn_readfirstlane((int)n);
+        if (n < size) return group_tile(g, dealt + n);
     }
     return tiles;
 }
 // Every block calls it once, after its last next_tile().
-__device__ __forceinline__ void tiles_done(TileWork* work, uint32_t tiles) {
-    if (gridDim.x >= tiles || (threadIdx.x & 63u) != 0) return;
+__device__ __forceinline__ void tiles_done(TileWork* work, uint32_t dealt) {
+    if (dealt == 0u || (threadIdx.x & 63u) != 0) return;
     const uint32_t g = blockIdx.x % kTileGroups;
-    if (atomicAdd(&work->done[g].v, 1u) != gridDim.x / kTileGroups - 1u) return;
+    if (atomicAdd(&work->done[g].v, 1u) != dealt - 1u) return;
     atomicExch(&work->done[g].v, 0u);
     if (atomicAdd(&work->groups.v, 1u) != kTileGroups - 1u) return;
     for (uint32_t k = 0; k < kTileGroups; ++k) atomicExch(&work->next[k].v, 0u);
