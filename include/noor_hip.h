@@ -323,7 +323,9 @@ noor_status noor_get_stats(noor_ctx* ctx, noor_stats* stats);
 noor_status noor_reset_stats(noor_ctx* ctx);
 noor_status noor_synchronize(noor_ctx* ctx);
 
-/* Closest-hit (any_hit = 0) or any-hit (any_hit = 1) queries on host arrays. */
+/* Closest-hit (any_hit = 0) or any-hit (any_hit = 1) queries on host arrays.
+ * The context keeps device memory for its largest call so far, up to 64 MiB (one
+ * million rays), until noor_destroy; larger calls allocate for themselves. */
 noor_status noor_trace(noor_ctx* ctx, const noor_ray* rays, uint32_t n, int any_hit,
                        noor_hit* hits);
 /* noor_trace without allocating: no counterpart in the reference; for callers

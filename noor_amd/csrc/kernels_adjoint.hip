@@ -33,7 +33,7 @@ struct AdjArgs {
     uint32_t stream;         // RNG stream (frame number) of the forward sample
 };
 
-// waves per SIMD: the box's 512x512 sample takes 0.80 ms, 0.92 at three, 0.98 at two
+// waves per SIMD: the box's 512x512 sample takes 0.78 ms, 0.93 at two, 0.88 at three, 0.87 at five
 constexpr int kAdjWaves = 4;
 constexpr uint32_t kLdsMats = 64;  // materials whose terms are summed in LDS first
 

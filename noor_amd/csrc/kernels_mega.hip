@@ -47,10 +47,11 @@ __device__ __forceinline__ void flush_stats(DevStats* st, unsigned long long ext
 // film (a separate instantiation keeps the film path's register budget).
 // Held to four waves per SIMD: the spills (outside the traversal's loop) cost less
 // than the waits that the third and fourth wave hide.  512x512x4 samples of the
-// box take 2.6 ms, 3.2 at two or three waves, 4.1 at five; the 1080p terrain frame
-// 3.0 ms, 4.6 at two, 3.1 at three and five.  Lanes that take the next sample or
-// pixel as soon as theirs ends, instead of with their wave, gain nothing (2.8 and
-// 3.0 ms): the mixed rays cost what the fuller waves save.
+// box take 2.28 ms, 3.1 at two waves, 3.0 at three, 2.6 at five; the 1080p terrain
+// frame 2.85 ms, 3.8 at two, 3.1 at three, 2.9 at five.  Lanes that take the next
+// sample or pixel as soon as theirs ends, instead of with their wave, gain nothing
+// (measured with 64-pixel tiles for every image: box 2.8 against 2.6 ms, terrain
+// equal): the mixed rays cost what the fuller waves save.
 // TEX: image textures, alpha tests, bump and ray differentials; two waves (256
 // VGPRs with spills already).
 constexpr int kMegaWaves = 4;

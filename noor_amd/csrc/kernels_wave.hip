@@ -419,10 +419,9 @@ __device__ __forceinline__ uint32_t refill(uint32_t* work, uint32_t count, bool 
     return !have && valid ? idx : 0xFFFFFFFFu;
 }
 
-// 79 VGPRs, six waves per SIMD, no spills: the traversal issues a VALU
-// instruction in nearly every slot (SQ_ACTIVE_INST_VALU at 97% of the SIMDs'
-// issue slots on the 1080p terrain), so its time follows the instructions of a
-// step.  At five waves the terrain film's k_extend takes 20.5 instead of 19.1
+// 80 VGPRs, six waves per SIMD, no spills: the traversal issues VALU
+// instructions without a gap (SQ_ACTIVE_INST_VALU: one per SIMD and four cycles
+// on the 1080p terrain), so its time follows the instructions of a step.  At five waves the terrain film's k_extend takes 20.5 instead of 19.1
 // ms, at seven (spills) 25.5.
 template <bool STATS, bool ALPHA>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_extend(

@@ -15,7 +15,7 @@ namespace noor {
 
 // The launch has at most as many blocks as the GPU holds at once; a block that
 // is done with its tile takes another one (with the tiles dealt out in advance
-// the 1080p terrain frame takes 3.6 instead of 3.0 ms).  The tiles are split
+// the 1080p terrain frame takes 3.5 instead of 2.85 ms).  The tiles are split
 // over kTileGroups groups with a counter each, block b taking from group
 // b % kTileGroups, one group per XCD: returning atomics on one address are
 // 11.7 ns apart, which with one counter made a frame whose rays all miss take
